@@ -8,6 +8,9 @@
 // (n = the segment's key count); for decode (L = 1) that is every key. A row with no visible key
 // outputs zeros. Softmax scale `scale`, accumulation in f32, output rounded to the input type.
 //
+// Calls with many query rows (prefill) run the kernel of attention_tile.hip; takes_tiles has the
+// rule. Here: decode, and a few query rows on a cached prefix.
+//
 // Work split (flash decoding): a workgroup of four waves owns R query rows of one segment and
 // one block of keys; each wave takes 12-16 KB of its K rows (wave_keys) and issues every load
 // (queries, K rows, V slices) before the first use, so one memory round trip covers the wave.
@@ -24,18 +27,11 @@
 #include <mutex>
 #include <string>
 
-#include "lr_common.hpp"
+#include "attention_tile.hpp"
 
 namespace lr {
 namespace {
 
-typedef __bf16 attn_bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 attn_f16x8 __attribute__((ext_vector_type(8)));
-typedef float attn_f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned attn_u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kAttnWaves = 4;
-constexpr int kAttnThreads = 64 * kAttnWaves;
 // Keys per wave: 12 KB of K rows (and as many V bytes) for d64/d128, 16 KB for d256 (a whole
 // number of 16-key MFMA blocks); small enough for three waves per SIMD. A call whose blocks of
 // that size would not give every CU two workgroups (batch-1 decode: cfg1 has 96) takes one
@@ -43,109 +39,13 @@ constexpr int kAttnThreads = 64 * kAttnWaves;
 constexpr int wave_keys(int dim) { return dim == 256 ? 32 : 6144 / dim; }
 constexpr int kSmallWaveKeys = 16;
 constexpr int64_t kFewBlocks = 512;
+// Partial states the allocation-free entry point holds (per device).
+constexpr size_t kAttentionScratchBytes = size_t{16} << 20;
 // Partial blocks each merging thread loads at once: four, or twelve where a thread folds more
 // than four blocks (batch-1 decode: cfg1's 36 blocks per unit take one round of loads instead
 // of three; measured 14.9 against 15.3 us per layer, and no better for cfg2's 12 blocks).
 constexpr int kMergeUnroll = 4;
 constexpr int kMergeUnrollWide = 12;
-constexpr float kAttnLog2e = 1.4426950408889634f;
-constexpr float kNegInf = -__builtin_huge_valf();
-
-template <typename T> struct AttnVec;
-template <> struct AttnVec<__bf16> {
-  using x8 = attn_bf16x8;
-  static __device__ __forceinline__ attn_f32x4 mfma(x8 a, x8 b, attn_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct AttnVec<_Float16> {
-  using x8 = attn_f16x8;
-  static __device__ __forceinline__ attn_f32x4 mfma(x8 a, x8 b, attn_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-struct AttnArgs {
-  const void* queries;      // element strides below; the last dimension is contiguous
-  int64_t q_batch, q_head, q_query;
-  const void* keys;         // [key_rows, D]
-  const void* values;       // [key_rows, D]
-  int64_t key_rows;
-  const int32_t* cu;        // [segments + 1]
-  int64_t kv_heads, groups, length;
-  int64_t tiles;            // query-row tiles per segment: ceil(L*G / R)
-  int64_t splits;           // key chunks per (segment, tile) in the grid
-  float scale;
-  void* out;                // [B, L, kv_heads * G, D]
-  float* part_o;            // [units * splits, R, D]
-  float* part_ml;           // [units * splits, R, 2]
-  const void* pending_keys;    // NULL, or [segments, D]: a row after each segment's cached rows
-  const void* pending_values;  // with pending_keys
-};
-
-template <typename T>
-__device__ __forceinline__ void unpack8(attn_u32x4 raw, float (&v)[8]) {
-  if constexpr (std::is_same<T, __bf16>::value) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[2 * e] = __builtin_bit_cast(float, raw[e] << 16);
-      v[2 * e + 1] = __builtin_bit_cast(float, raw[e] & 0xffff0000u);
-    }
-  } else {
-    const attn_f16x8 h = __builtin_bit_cast(attn_f16x8, raw);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h[e]);
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ attn_u32x4 pack8(const float (&v)[8]) {
-  typename AttnVec<T>::x8 h;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) h[e] = static_cast<T>(v[e]);  // round to nearest even
-  return __builtin_bit_cast(attn_u32x4, h);
-}
-
-__device__ __forceinline__ attn_u32x4 load16(const void* p) {
-  return *(const __attribute__((address_space(1))) attn_u32x4*)p;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1) v = fmaxf(v, __shfl_xor(v, offset));
-  return v;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset);
-  return v;
-}
-
-// Output row `row` of segment `seg` (query i = row / G, query head h*G + row % G).
-template <typename T, int D>
-__device__ __forceinline__ T* output_row(const AttnArgs& a, int64_t seg, int64_t row) {
-  const int64_t b = seg / a.kv_heads, h = seg - b * a.kv_heads;
-  const int64_t i = row / a.groups, g = row - i * a.groups;
-  const int64_t heads = a.kv_heads * a.groups;
-  return static_cast<T*>(a.out) + ((b * a.length + i) * heads + h * a.groups + g) * D;
-}
-
-// A (max, exp-sum, unnormalised output slice) softmax state; merge_into folds another in.
-struct MergeState {
-  float m, l, o[8];
-};
-
-__device__ __forceinline__ void merge_into(MergeState& s, float m, float l, const float (&o)[8]) {
-  if (m == kNegInf) return;
-  const float mx = fmaxf(s.m, m);
-  const float ws = s.m == kNegInf ? 0.f : __builtin_amdgcn_exp2f((s.m - mx) * kAttnLog2e);
-  const float wo = __builtin_amdgcn_exp2f((m - mx) * kAttnLog2e);
-  s.l = __builtin_fmaf(wo, l, s.l * ws);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) s.o[e] = __builtin_fmaf(wo, o[e], s.o[e] * ws);
-  s.m = mx;
-}
 
 template <typename T, int D, int R, int CH>
 __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attention_kernel(AttnArgs a) {
@@ -484,6 +384,28 @@ size_t workspace_bytes(const AttnPlan& p, int64_t dim) {
   return static_cast<size_t>(slots) * static_cast<size_t>(dim + 2) * 4;
 }
 
+// Whether a call runs the prefill kernel (attention_tile.hip). The split-key kernel stays for
+// decode, and for the few rows a 32-row tile would leave mostly empty: up to 32 rows on a cached
+// prefix (d128, G4: 2 queries on 500 keys 10.9 us against 12.5, 8 queries on 4000 keys 23.2
+// against 25.0), while the segments' keys fit one round of its blocks (3 x 8 segments of 2,861
+// keys, 8 queries: 35.1 against 23.1 us). At d64 the tiles are already ahead (2 queries on 500
+// keys 9.1 against 11.5 us, 8 on 4000 14.9 against 32.8).
+bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys, int64_t dim) {
+  if (length <= 1 || length > INT32_MAX / groups) return false;
+  const bool few_rows = length * groups <= 32;
+  return dim == 64 || !few_rows || max_keys <= 128 || max_keys > 40000 / segments;
+}
+
+// The prefill kernel's plan. Its partial states stay within the allocation-free entry point's
+// array for every call that entry point accepts (its limit is the split-key plan's bytes, below),
+// and within 32 MiB otherwise.
+AttnTilePlan plan_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys,
+                        int64_t dim) {
+  const size_t blocks = workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim);
+  const size_t most = blocks <= kAttentionScratchBytes ? kAttentionScratchBytes : size_t{32} << 20;
+  return plan_attention_tiles(segments, groups, length, max_keys, dim, static_cast<int64_t>(most));
+}
+
 template <typename T, int D, int R, int CH>
 int launch_attention(const AttnArgs& args, int64_t blocks, hipStream_t stream) {
   hipLaunchKernelGGL((packed_attention_kernel<T, D, R, CH>), dim3(static_cast<unsigned>(blocks)),
@@ -535,23 +457,21 @@ extern "C" size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t 
                                                       int64_t length, int64_t max_keys,
                                                       int64_t dim) {
   if (segments <= 0 || groups <= 0 || length <= 0 || max_keys < 0 || dim <= 0) return 0;
+  if (takes_tiles(segments, groups, length, max_keys, dim))
+    return attention_tiles_bytes(plan_tiles(segments, groups, length, max_keys, dim), dim);
   return workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim);
 }
 
 namespace lr {
 namespace {
 
-// The checks and launches shared by lr_packed_attention and lr_packed_attention_noalloc.
-// `scratch_limit` is nonzero for the allocation-free variant: its workspace is the library's
-// fixed per-device array of that size, and a call that needs more is refused with its own
-// message before anything is enqueued.
+// The checks and launches shared by the entry points.
 int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head_stride,
                      int64_t q_query_stride, const void* keys, const void* values,
                      int64_t key_rows, const int32_t* cu_seqlens_k, int64_t batch,
                      int64_t kv_heads, int64_t groups, int64_t length, int64_t dim, int dtype,
                      int64_t max_keys, float scale, void* out, void* workspace,
-                     size_t workspace_size, size_t scratch_limit, void* stream,
-                     const void* pending_keys = nullptr, const void* pending_values = nullptr) {
+                     size_t workspace_size, void* stream, const void* pending_keys = nullptr, const void* pending_values = nullptr) {
   LR_REQUIRE(dtype == LR_DTYPE_BF16 || dtype == LR_DTYPE_F16,
              "FlashAttention only supports fp16 and bf16 data type");
   LR_REQUIRE((pending_keys == nullptr) == (pending_values == nullptr),
@@ -574,13 +494,11 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
   const int64_t segments = batch * kv_heads;
   if (pending_keys != nullptr) ++max_keys;  // every segment's pending row
   const AttnPlan plan = plan_attention(segments, groups, length, max_keys, dim);
-  const size_t needed = workspace_bytes(plan, dim);
-  if (scratch_limit) {
-    LR_REQUIRE(needed <= scratch_limit,
-               "Attention needs " + std::to_string(needed) +
-                   " bytes of scratch; the allocation-free entry point holds at most " +
-                   std::to_string(scratch_limit) + " bytes per device");
-  }
+  const bool use_tiles = takes_tiles(segments, groups, length, max_keys, dim);
+  AttnTilePlan tile_plan{};
+  if (use_tiles) tile_plan = plan_tiles(segments, groups, length, max_keys, dim);
+  const size_t needed =
+      use_tiles ? attention_tiles_bytes(tile_plan, dim) : workspace_bytes(plan, dim);
   LR_REQUIRE(workspace_size >= needed && (needed == 0 || workspace != nullptr),
              "Attention workspace too small");
   LR_REQUIRE(needed == 0 || reinterpret_cast<uintptr_t>(workspace) % 256 == 0,
@@ -606,11 +524,20 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
   args.out = out;
   args.pending_keys = pending_keys;
   args.pending_values = pending_values;
+  const hipStream_t s = as_stream(stream);
+  if (use_tiles) {
+    args.tiles = tile_plan.tiles;
+    args.splits = tile_plan.splits;
+    if (needed) {
+      args.part_ml = static_cast<float*>(workspace);
+      args.part_o = args.part_ml + segments * tile_plan.tiles * tile_plan.splits * tile_plan.rows * 2;
+    }
+    return launch_attention_tiles(args, tile_plan, dim, dtype, s);
+  }
   if (needed) {
     args.part_ml = static_cast<float*>(workspace);
     args.part_o = args.part_ml + plan.units * plan.splits * plan.rows_per_tile * 2;
   }
-  const hipStream_t s = as_stream(stream);
   return dtype == LR_DTYPE_BF16
              ? launch_dim<__bf16>(args, dim, plan, blocks, s)
              : launch_dim<_Float16>(args, dim, plan, blocks, s);
@@ -620,7 +547,6 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
 // library's load onto that device until the process ends. Host code never passes `scratch`
 // itself to a kernel (on the host the name is only a stand-in for the symbol); it passes the
 // device address hipGetSymbolAddress gives, looked up once per device.
-constexpr size_t kAttentionScratchBytes = size_t{16} << 20;
 __device__ __align__(256) unsigned char scratch[kAttentionScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -670,7 +596,7 @@ extern "C" int lr_packed_attention(const void* queries, int64_t q_batch_stride,
   clear_error();
   return packed_attention(queries, q_batch_stride, q_head_stride, q_query_stride, keys, values,
                           key_rows, cu_seqlens_k, batch, kv_heads, groups, length, dim, dtype,
-                          max_keys, scale, out, workspace, workspace_size, 0, stream);
+                          max_keys, scale, out, workspace, workspace_size, stream);
 }
 
 extern "C" size_t lr_packed_attention_pending_workspace_bytes(int64_t segments, int64_t groups,
@@ -691,8 +617,7 @@ extern "C" int lr_packed_attention_pending(const void* queries, int64_t q_batch_
   LR_REQUIRE(pending_keys != nullptr && pending_values != nullptr, "Invalid attention buffers");
   return packed_attention(queries, q_batch_stride, q_head_stride, q_query_stride, keys, values,
                           key_rows, cu_seqlens_k, batch, kv_heads, groups, 1, dim, dtype,
-                          max_keys, scale, out, workspace, workspace_size, 0, stream,
-                          pending_keys, pending_values);
+                          max_keys, scale, out, workspace, workspace_size, stream, pending_keys, pending_values);
 }
 
 extern "C" size_t lr_packed_attention_scratch_bytes(void) { return kAttentionScratchBytes; }
@@ -710,11 +635,16 @@ extern "C" int lr_packed_attention_noalloc(const void* queries, int64_t q_batch_
   // (every segment within one key block) does not touch the scratch array at all.
   const int64_t segments =
       batch > 0 && kv_heads > 0 && batch <= (int64_t{1} << 31) / kv_heads ? batch * kv_heads : 0;
-  const size_t needed = lr_packed_attention_workspace_bytes(segments, groups, length, max_keys, dim);
-  LR_REQUIRE(needed <= kAttentionScratchBytes,
-             "Attention needs " + std::to_string(needed) +
+  // The limit is stated in the split-key plan's bytes whichever kernels run (plan_tiles keeps the
+  // prefill kernel's partial states of an accepted call within the array).
+  const bool sized = segments > 0 && groups > 0 && length > 0 && max_keys >= 0 && dim > 0;
+  const size_t blocks =
+      sized ? workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim) : 0;
+  LR_REQUIRE(blocks <= kAttentionScratchBytes,
+             "Attention needs " + std::to_string(blocks) +
                  " bytes of scratch; the allocation-free entry point holds at most " +
                  std::to_string(kAttentionScratchBytes) + " bytes per device");
+  const size_t needed = lr_packed_attention_workspace_bytes(segments, groups, length, max_keys, dim);
   void* workspace = nullptr;
   if (needed) {
     if (int status = scratch_address(as_stream(stream), &workspace)) return status;
@@ -722,5 +652,5 @@ extern "C" int lr_packed_attention_noalloc(const void* queries, int64_t q_batch_
   return packed_attention(queries, q_batch_stride, q_head_stride, q_query_stride, keys, values,
                           key_rows, cu_seqlens_k, batch, kv_heads, groups, length, dim, dtype,
                           max_keys, scale, out, workspace, needed ? kAttentionScratchBytes : 0,
-                          kAttentionScratchBytes, stream);
+                          stream);
 }

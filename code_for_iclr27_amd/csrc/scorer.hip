@@ -25,6 +25,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "lds_copy.hpp"
 #include "lr_common.hpp"
 
 namespace lr {
@@ -297,108 +298,6 @@ __global__ __launch_bounds__(256) void projected_values_kernel(const int64_t* __
     reduce(first, cur);
 #pragma unroll
     for (int k = 0; k < kRows; ++k) cur[k] = next[k];
-  }
-}
-
-// Direct global -> LDS copies (global_load_lds_dword / _dwordx4): lane L of a wave writes its
-// granule at LDS `wave_base` + L * granule; `wave_base` must be the same for the whole wave.
-// Nothing passes through VGPRs. Completion is awaited with dma_wait() before the barrier that
-// publishes the data.
-// The copies are issued by inline assembly, not by the compiler's builtin: for the builtin the
-// compiler makes every later LDS read that it cannot prove disjoint from the copy wait for it
-// (s_waitcnt vmcnt(0)), and a buffer picked at run time is never provably disjoint, so the
-// copy of the next stage would be waited for at the first read of the current one. Copies the
-// compiler does not see only lengthen its own vmcnt waits (counts drain in order), never
-// shorten them. M0 (the wave's LDS base for the copy) is set inside the same statement; no
-// compiler-generated code in these kernels keeps a value in M0.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // M0 is a reserved register; clobbered on purpose
-// Copy from a per-lane address to the (wave-uniform) LDS byte address `lds`.
-__device__ __forceinline__ void dma16_to(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(src), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4_to(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-               :: "v"(src), "s"(lds) : "memory", "m0");
-}
-// The same copies addressed as a wave-uniform base (an SGPR pair) plus a per-lane 32-bit byte
-// offset: the per-copy address arithmetic is then scalar, and a lane's offset can be computed
-// once.
-__device__ __forceinline__ void dma16_at(const void* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4_at(const void* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-               :: "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// LDS byte address of a __shared__ object.
-template <typename T>
-__device__ __forceinline__ uint32_t lds_address(T* object) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) T*)object));
-}
-
-__device__ __forceinline__ uint32_t wave_index() {
-  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-}
-
-// vmcnt(0) through the builtin, so that the compiler knows every vector-memory load has landed
-// here (loads issued before a loop, such as the resident MFMA operands, are then not waited for
-// again inside it); the empty statement keeps LDS accesses from moving across the wait.
-__device__ __forceinline__ void dma_wait() {
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-  asm volatile("" ::: "memory");
-}
-
-// Swizzled LDS rows: D bf16 per row, no padding; 16-byte chunk c of row r is stored in chunk
-// slot c ^ (r % P), so the lanes that read chunk c of consecutive rows (an MFMA operand) touch
-// P different 16-byte bank groups per P rows. P = 16 for d = 128 (its 16 chunks per row allow
-// it; measured 2% faster in the row pass than P = 8), else 8.
-template <int D>
-constexpr int swizzle_period() { return D == 128 ? 16 : 8; }
-
-template <int D>
-__device__ __forceinline__ int swizzled_chunk(int row, int chunk) {
-  return chunk ^ (row & (swizzle_period<D>() - 1));
-}
-
-// DMA of `ROWS` consecutive rows (row0..) of a [*, D] bf16 matrix into swizzled LDS rows at LDS
-// byte address `lds`; rows at or past `last_row` re-read row `last_row` (callers mask them). All
-// 256 threads call it. Copy i moves rows [i * RPI, (i + 1) * RPI), RPI = 256 / (D / 8), a
-// multiple of the swizzle period, so a thread's (row % RPI, chunk) and hence its swizzled byte
-// offset within the copy (`dma_row_offset`) are the same for every i: while every row lies
-// before `last_row` the addresses are a scalar base plus that fixed offset.
-template <int D>
-__device__ __forceinline__ uint32_t dma_row_offset() {
-  constexpr int CH = D / 8;
-  const int row = threadIdx.x / CH, chunk = threadIdx.x % CH;
-  return static_cast<uint32_t>((row * D + 8 * swizzled_chunk<D>(row, chunk)) * 2);
-}
-
-template <int D, int ROWS>
-__device__ __forceinline__ void dma_rows(const __bf16* matrix, int row0, int last_row,
-                                         uint32_t lds, uint32_t row_offset) {
-  constexpr int CH = D / 8, CHUNKS = ROWS * CH, RPI = 256 / CH;
-  static_assert(CHUNKS % 256 == 0 && RPI % swizzle_period<D>() == 0,
-                "whole waves per copy, whole swizzle periods");
-  const uint32_t wave_lds = lds + wave_index() * 64 * 16;
-  if (row0 + ROWS - 1 <= last_row) {
-    const char* base = reinterpret_cast<const char*>(matrix + static_cast<int64_t>(row0) * D);
-#pragma unroll
-    for (int i = 0; i < CHUNKS / 256; ++i)
-      dma16_at(base + static_cast<int64_t>(i) * RPI * D * 2, row_offset, wave_lds + 256 * 16 * i);
-  } else {
-#pragma unroll
-    for (int i = 0; i < CHUNKS / 256; ++i) {
-      const int slot = 256 * i + threadIdx.x;
-      const int row = slot / CH, chunk = slot % CH;
-      const int source = min(row0 + row, last_row);
-      dma16_to(matrix + static_cast<int64_t>(source) * D + 8 * swizzled_chunk<D>(row, chunk),
-               wave_lds + 256 * 16 * i);
-    }
   }
 }
 

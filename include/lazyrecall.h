@@ -461,9 +461,9 @@ int lr_history_append(const void* const* layer_queries, int64_t layers, int64_t 
  * with no visible key is zero. out is [batch, length, kv_heads*groups, dim] contiguous, of the
  * input dtype (LR_DTYPE_BF16 or LR_DTYPE_F16); dim in {64, 128, 256}. max_keys bounds every
  * segment's key count (keys past it are not read). workspace: device scratch of at least
- * lr_packed_attention_workspace_bytes(...) bytes (0 when every segment fits one block of keys),
- * 256-byte aligned, no initial contents required; calls that overlap in time need their own.
- * Two launches when a segment spans several key blocks (blocks, then their merge). */
+ * lr_packed_attention_workspace_bytes(...) bytes (0 when no segment's keys are split over
+ * workgroups), 256-byte aligned, no initial contents required; calls that overlap in time need
+ * their own. Two launches when they are split (key blocks, then their merge). */
 size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t groups, int64_t length,
                                            int64_t max_keys, int64_t dim);
 int lr_packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head_stride,
@@ -498,9 +498,11 @@ int lr_packed_attention_pending(const void* queries, int64_t q_batch_stride,
  * that forbid hipMalloc). Same arguments, kernels and results as lr_packed_attention, without
  * the workspace: the partial states live in one fixed array per device of
  * lr_packed_attention_scratch_bytes() bytes (16 MiB), held from the library's first use on that
- * device until the process ends. The call allocates and frees nothing. A call whose
- * lr_packed_attention_workspace_bytes(...) exceeds that size returns LR_ERR_INVALID with a
- * message naming both sizes, before anything is enqueued. Every call on one device shares that
+ * device until the process ends. The call allocates and frees nothing. A call whose keys, split
+ * as a decode call splits them (192 to 768 keys and up to 8 query rows a partial state), would
+ * leave more than that size of partial states returns LR_ERR_INVALID with a message naming both
+ * sizes, before anything is enqueued; prefill kernels keep theirs within it for every call
+ * accepted. Every call on one device shares that
  * device's array and leaves its contents behind (none are needed at the next call): two calls
  * that can overlap in time on one device (different streams without an order between them)
  * race on it. The device is the one that owns `stream` (the current device for NULL). */

@@ -108,6 +108,74 @@ def test_long_prefill_many_chunks(device):
     check(run(device, q, k, v, meta, length, 1), q, k, v, cu, 1)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,kv_heads,groups,length,dim,lengths", [
+    (1, 2, 3, 11, 128, [11, 43]),                    # 33 rows: a 32-row tile and one row more
+    (1, 2, 1, 32, 64, [32, 33]),                     # one whole tile; a last stage of one key
+    (2, 1, 5, 26, 256, [26, 31]),                    # 130 rows
+    (1, 3, 4, 40, 64, [1040, 40, 7]),                # split keys; a segment shorter than the block
+    (1, 2, 4, 40, 128, [2040, 0]),                   # split keys; an empty segment
+    (1, 4, 6, 64, 256, [1064, 64, 300, 2064]),       # split keys, ragged
+    (2, 8, 8, 256, 128, [256] * 15 + [611]),         # tiles of 128 rows
+    (2, 8, 8, 256, 64, [256] * 15 + [300]),
+    (2, 6, 7, 131, 256, [131] * 11 + [700]),         # 917 rows: a ragged last tile
+    (1, 1, 4, 300, 128, [4300]),                     # few units, long keys: many chunks
+])
+def test_prefill_tiles(device, dtype, batch, kv_heads, groups, length, dim, lengths):
+    """The prefill kernel at the edges of its 32- and 128-row tiles, its 32-key stages and its key
+    chunks, and on segments with fewer keys than queries."""
+    q, k, v, cu, meta = make(device, batch, kv_heads, groups, length, dim, lengths, dtype, seed=17)
+    check(run(device, q, k, v, meta, length, kv_heads), q, k, v, cu, kv_heads)
+
+
+@pytest.mark.parametrize("dim,groups,history", [(64, 4, 0), (128, 4, 700), (256, 2, 40)])
+def test_prefill_masked_keys_never_contribute(device, dim, groups, history):
+    """A NaN and an infinity in V at one key: rows that do not see it are those of the finite V
+    (within the tolerance), rows that do are not finite in its columns and unchanged in others."""
+    length, kv_heads, at = 90, 2, history + 41
+    q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim,
+                             [history + length] * kv_heads, seed=18)
+    finite = run(device, q, k, v, meta, length, kv_heads)
+    check(finite, q, k, v, cu, kv_heads)
+    bad = v.clone()
+    bad[at, 3], bad[at, dim - 1] = float("nan"), float("inf")
+    got = run(device, q, k, bad, meta, length, kv_heads).view(length, kv_heads, groups, dim)
+    finite = finite.view(length, kv_heads, groups, dim)
+    columns = torch.tensor([3, dim - 1], device=device)
+    seen = at - history
+    assert not torch.isfinite(got[seen:, 0][..., columns]).any()
+    changed = torch.zeros_like(got, dtype=torch.bool)
+    changed[seen:, 0] = torch.isin(torch.arange(dim, device=device), columns)
+    bound = ULP[got.dtype] * finite.float().abs() * 2 + 2e-4 * float(v.float().abs().max())
+    assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.125, 0.5])
+def test_prefill_scales_through_the_abi(device, scale):
+    """lr_packed_attention's scale is any number: zero (the mean of the visible values) and
+    negative ones too. A larger scale has a larger relative rounding of the f32 exponent, so
+    0.5 at d64 (logits up to 20) still fits the same tolerance."""
+    from code_for_iclr27_amd import _lib
+    length, kv_heads, groups, dim = 50, 2, 4, 64
+    q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim, [50, 120], seed=19)
+    tensors = [t.to(device) for t in (q, k, v)]
+    out = torch.empty((1, length, kv_heads * groups, dim), dtype=q.dtype, device=device)
+    size = _lib.load().lr_packed_attention_workspace_bytes(kv_heads, groups, length, 120, dim)
+    workspace = torch.empty(max(size, 256), dtype=torch.uint8, device=device)
+    for entry, extra in (("lr_packed_attention", [workspace.data_ptr(), workspace.numel()]),
+                         ("lr_packed_attention_noalloc", [])):
+        out.fill_(float("nan"))
+        _lib.call(entry, tensors[0].data_ptr(), *tensors[0].stride()[:3], tensors[1].data_ptr(),
+                  tensors[2].data_ptr(), k.shape[0], meta.cu_seqlens_k.data_ptr(), 1, kv_heads,
+                  groups, length, dim, _lib.LR_DTYPE_BF16, 120, scale, out.data_ptr(), *extra,
+                  torch.cuda.current_stream().cuda_stream)
+        expect = oattention.packed_attention(q.float().numpy(), k.float().numpy(),
+                                             v.float().numpy(), cu, kv_heads, scale)
+        error = np.abs(out.view(1, length, -1).float().cpu().numpy() - expect)
+        bound = ULP[q.dtype] * np.abs(expect) + 1e-4 * float(v.float().abs().max())
+        assert np.all(error <= bound)
+
+
 def test_strided_queries_as_the_reference_builds_them(device):
     # q_proj(x).view(B, L, Hq, d).transpose(1, 2): a non-contiguous [B, Hq, L, d] view.
     g = torch.Generator().manual_seed(12)
