@@ -54,11 +54,27 @@ __device__ __forceinline__ uint32_t wave_index() {
   return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
+// A wave-uniform address in scalar registers, also where the compiler formed it in vector ones.
+__device__ __forceinline__ const char* uniform_address(const void* p) {
+  const uint64_t bits = reinterpret_cast<uint64_t>(p);
+  const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits));
+  const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32));
+  return reinterpret_cast<const char*>(static_cast<uint64_t>(high) << 32 | low);
+}
+
 // vmcnt(0) through the builtin, so that the compiler knows every vector-memory load has landed
 // here (loads issued before a loop, such as the resident MFMA operands, are then not waited for
 // again inside it); the empty statement keeps LDS accesses from moving across the wait.
 __device__ __forceinline__ void dma_wait() {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
+  asm volatile("" ::: "memory");
+}
+
+// The same, leaving the `N` newest of the wave's vector-memory operations in flight.
+template <int N>
+__device__ __forceinline__ void dma_wait_but() {
+  static_assert(N >= 0 && N <= 63, "vmcnt holds six bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));  // vmcnt(N)
   asm volatile("" ::: "memory");
 }
 
@@ -89,39 +105,39 @@ struct ColumnSwizzle {
   static __device__ __forceinline__ int slot(int row, int chunk) { return chunk ^ (block(row) << 2); }
 };
 
-// DMA of `ROWS` consecutive rows (row0..) of a [*, D] 16-bit matrix into swizzled LDS rows at LDS
-// byte address `lds`; rows at or past `last_row` re-read row `last_row` (callers mask them). All
-// THREADS threads of the workgroup call it. Copy i moves rows [i * RPI, (i + 1) * RPI), RPI =
+// DMA of `ROWS` consecutive rows (row0..) of a 16-bit matrix, D elements of each (`stride` elements
+// from row to row: D, or a multiple of 128), into swizzled LDS rows at LDS byte address `lds`; rows at or past `last_row` re-read row `last_row` (callers mask them; no CLAMP: there are none). All
+// THREADS threads of the workgroup call it, or, with 64, one wave (with its lane as `thread`). Copy i moves rows [i * RPI, (i + 1) * RPI), RPI =
 // THREADS / (D / 8): while every row lies before `last_row` the addresses are a scalar base plus
 // the thread's byte offset within copy 0 (`dma_row_offset`), its chunk exchanged with what the
 // swizzle does to row i * RPI (nothing where RPI is a multiple of the swizzle's period).
 template <int D, typename Swizzle = RowSwizzle<D>, int THREADS = 256>
-__device__ __forceinline__ uint32_t dma_row_offset() {
+__device__ __forceinline__ uint32_t dma_row_offset(int thread = threadIdx.x, int stride = D) {
   constexpr int CH = D / 8;
-  const int row = threadIdx.x / CH, chunk = threadIdx.x % CH;
-  return static_cast<uint32_t>((row * D + 8 * Swizzle::slot(row, chunk)) * 2);
+  const int row = thread / CH, chunk = thread % CH;
+  return static_cast<uint32_t>((row * stride + 8 * Swizzle::slot(row, chunk)) * 2);
 }
 
-template <int D, int ROWS, typename Swizzle = RowSwizzle<D>, int THREADS = 256>
+template <int D, int ROWS, typename Swizzle = RowSwizzle<D>, int THREADS = 256, bool CLAMP = true>
 __device__ __forceinline__ void dma_rows(const __bf16* matrix, int row0, int last_row,
-                                         uint32_t lds, uint32_t row_offset) {
+                                         uint32_t lds, uint32_t row_offset, int stride = D) {
   constexpr int CH = D / 8, CHUNKS = ROWS * CH, RPI = THREADS / CH;
   static_assert(CHUNKS % THREADS == 0 && THREADS % CH == 0, "whole copies of whole rows");
   const uint32_t wave_lds = lds + (THREADS == 64 ? 0 : wave_index() * 64 * 16);
-  if (row0 + ROWS - 1 <= last_row) {
-    const char* base = reinterpret_cast<const char*>(matrix + static_cast<int64_t>(row0) * D);
+  if (!CLAMP || row0 + ROWS - 1 <= last_row) {
+    const char* base = uniform_address(matrix + static_cast<int64_t>(row0) * stride);
 #pragma unroll
     for (int i = 0; i < CHUNKS / THREADS; ++i)
-      dma16_at(base + static_cast<int64_t>(i) * RPI * D * 2,
+      dma16_at(base + static_cast<int64_t>(i) * RPI * stride * 2,
                row_offset ^ (16 * static_cast<uint32_t>(Swizzle::slot(i * RPI, 0))),
                wave_lds + THREADS * 16 * i);
   } else {
 #pragma unroll
     for (int i = 0; i < CHUNKS / THREADS; ++i) {
-      const int slot = THREADS * i + threadIdx.x;
+      const int slot = THREADS * i + (THREADS == 64 ? threadIdx.x & 63 : threadIdx.x);
       const int row = slot / CH, chunk = slot % CH;
       const int source = min(row0 + row, last_row);
-      dma16_to(matrix + static_cast<int64_t>(source) * D + 8 * Swizzle::slot(row, chunk),
+      dma16_to(matrix + static_cast<int64_t>(source) * stride + 8 * Swizzle::slot(row, chunk),
                wave_lds + THREADS * 16 * i);
     }
   }

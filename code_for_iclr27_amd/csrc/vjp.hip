@@ -7,6 +7,7 @@
 // from HBM once, in its own dtype (bf16/f16/f32), and does the arithmetic in f32 as the
 // reference's `.float()` GEMMs do; the reference instead materialises f32 copies of 4096-row
 // weight chunks (written and re-read) and the [rows, V] probability matrix.
+// Several rows against a bf16 weight run on matrix cores instead (vjp_products.hip).
 //   head_logits_kernel   Y[r, v] = sum_d X[r, d] * W[v, d] (+ b[v]); a wave owns 4 rows of W,
 //                        lanes split D (16 B loads), X staged in LDS, one wave reduction per row.
 //   margin stats         per logits row: target (given, or the first argmax), competitor max M,
@@ -23,6 +24,7 @@
 #include <algorithm>
 
 #include "lr_common.hpp"
+#include "vjp_products.hpp"
 
 namespace lr {
 namespace {
@@ -36,6 +38,7 @@ constexpr int kLogitRowsPerBlock = kLogitRowsPerWave * (kLogitThreads / 64);
 constexpr int kLogitLdsFloats = 16384;  // X rows staged per launch: rows * D <= this (64 KB)
 constexpr int kReduceThreads = 1024;
 constexpr int kReduceColumns = 64;
+constexpr int kReduceGroups = kReduceThreads / kReduceColumns;
 
 // Eight consecutive elements of a weight row as f32.
 template <typename T>
@@ -75,13 +78,17 @@ __global__ __launch_bounds__(kLogitThreads) void head_logits_kernel(
     const T* __restrict__ bias, int64_t vocab, float* __restrict__ out, int64_t out_stride) {
   extern __shared__ __align__(16) float x[];  // [RP, dim]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  for (int64_t i = tid; i < RP * dim; i += kLogitThreads) {
-    const int64_t r = i / dim;
-    x[i] = r < rows_here ? hidden[i] : 0.f;
-  }
+#pragma unroll
+  for (int r = 0; r < RP; ++r)
+    for (int64_t i = tid; i < dim; i += kLogitThreads)
+      x[r * dim + i] = r < rows_here ? hidden[r * dim + i] : 0.f;
   __syncthreads();
   const int64_t chunks = dim / 8;
-  const int64_t v0 = static_cast<int64_t>(blockIdx.x) * kLogitRowsPerBlock + wave * kLogitRowsPerWave;
+  // Several rows: as many blocks as fit the chip, each staging X once for all its rows of W (a
+  // block per 16 rows of W stages half as many bytes of X again: eight f16 rows of 128,256 x 4096
+  // take 475 us against 967). One row: a block per 16 rows of W (188 against 217 us in a loop).
+  for (int64_t block = blockIdx.x; block * kLogitRowsPerBlock < vocab; block += gridDim.x) {
+  const int64_t v0 = block * kLogitRowsPerBlock + wave * kLogitRowsPerWave;
   const T* wrow[kLogitRowsPerWave];
 #pragma unroll
   for (int i = 0; i < kLogitRowsPerWave; ++i) {
@@ -125,6 +132,8 @@ __global__ __launch_bounds__(kLogitThreads) void head_logits_kernel(
       for (int r = 0; r < RP; ++r)
         if (r < rows_here) out[r * out_stride + v] = bias ? acc[i][r] + b : acc[i][r];
     }
+  }
+  if constexpr (RP == 1) return;
   }
 }
 
@@ -312,10 +321,7 @@ struct RowSumArgs {
   const float* stats;
   const int64_t* targets;
   const float* coefficients;
-  float* partial;             // [blocks, rows, dim] (per layer with a layer table)
-  // Several weights in one launch (blockIdx.z = layer): device [layers, 4] words (weight,
-  // coefficients, gate or 0, out); weight and coefficients above are then unused.
-  const int64_t* layer_table;
+  float* partial;             // [blocks, rows, dim]
 };
 
 // grid: (ceil(dim / 2048) column blocks, ceil(vocab / rows_per_block) row blocks) of 256
@@ -329,15 +335,6 @@ template <typename T, int RP>
 __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
   extern __shared__ float coef[];  // [rows_per_block][RP]
   const int tid = threadIdx.x;
-  const void* weight_ptr = a.weight;
-  const float* coefficients = a.coefficients;
-  float* partial = a.partial;
-  if (a.layer_table) {
-    const int64_t* entry = a.layer_table + 4 * static_cast<int64_t>(blockIdx.z);
-    weight_ptr = reinterpret_cast<const void*>(entry[0]);
-    coefficients = reinterpret_cast<const float*>(entry[1]);
-    partial += static_cast<int64_t>(blockIdx.z) * gridDim.y * a.rows * a.dim;
-  }
   const int64_t v0 = static_cast<int64_t>(blockIdx.y) * a.rows_per_block;
   const int64_t count = a.vocab - v0 < a.rows_per_block ? a.vocab - v0 : a.rows_per_block;
   for (int64_t i = tid; i < a.rows_per_block * RP; i += kRowSumThreads) {
@@ -349,7 +346,7 @@ __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
         c = v == a.targets[r] ? 0.f
                               : expf(a.logits[r * a.vocab + v] - a.stats[2 * r]) / a.stats[2 * r + 1];
       } else {
-        c = coefficients[r * a.vocab + v];
+        c = a.coefficients[r * a.vocab + v];
       }
     }
     coef[i] = c;
@@ -357,7 +354,7 @@ __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
   __syncthreads();
   const int64_t col = static_cast<int64_t>(blockIdx.x) * kRowSumColumns + 8 * tid;
   if (col >= a.dim) return;  // no barrier follows
-  const T* weight = static_cast<const T*>(weight_ptr);
+  const T* weight = static_cast<const T*>(a.weight);
   float acc[RP][8];
 #pragma unroll
   for (int r = 0; r < RP; ++r)
@@ -389,11 +386,59 @@ __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
       for (int e = 0; e < 8; ++e) acc[r][e] = __builtin_fmaf(c, w[e], acc[r][e]);
     }
   }
-  for (int r = 0; r < RP && r < a.rows; ++r) {
-    float* p = partial + (static_cast<int64_t>(blockIdx.y) * a.rows + r) * a.dim + col;
+#pragma unroll
+  for (int r = 0; r < RP; ++r) {  // unrolled: indexed at run time, acc would live in memory
+    if (r >= a.rows) break;
+    float* p = a.partial + (static_cast<int64_t>(blockIdx.y) * a.rows + r) * a.dim + col;
     *reinterpret_cast<vjp_f32x4*>(p) = vjp_f32x4{acc[r][0], acc[r][1], acc[r][2], acc[r][3]};
     *reinterpret_cast<vjp_f32x4*>(p + 4) = vjp_f32x4{acc[r][4], acc[r][5], acc[r][6], acc[r][7]};
   }
+}
+
+// One coefficient row for each of several weights (pre-projection gradients of every layer).
+// grid: (column blocks, reduction groups, layers) of 256 threads, device [layers, 4] words (weight,
+// coefficients, gate or 0, out). A workgroup takes every row block b with b % groups = its group,
+// sums each as row_sum_kernel does and adds the sums in block order, as row_sum_reduce_kernel adds
+// its group: the same result bit for bit, with one partial row a group instead of one a block
+// (32 x 4096 x 4096 bf16: 8 MB of partials instead of 67 MB each way; 188 us instead of 223).
+template <typename T>
+__global__ __launch_bounds__(kRowSumThreads) void row_sum_layers_kernel(
+    const int64_t* __restrict__ layer_table, int64_t vocab, int64_t dim, int64_t block_rows,
+    int64_t blocks, float* __restrict__ partial) {
+  const int64_t* entry = layer_table + 4 * static_cast<int64_t>(blockIdx.z);
+  const T* weight = reinterpret_cast<const T*>(entry[0]);
+  const float* coefficients = reinterpret_cast<const float*>(entry[1]);
+  const int64_t group = blockIdx.y, groups = gridDim.y;
+  const int64_t col = static_cast<int64_t>(blockIdx.x) * kRowSumColumns + 8 * threadIdx.x;
+  if (col >= dim) return;
+  float total[8] = {};
+  for (int64_t b = group; b < blocks; b += groups) {
+    const int64_t v0 = b * block_rows;
+    const float* c = coefficients + v0;  // the same for every thread: scalar loads
+    const int64_t count = vocab - v0 < block_rows ? vocab - v0 : block_rows;
+    float acc[8] = {};
+    int64_t k = 0;
+    for (; k + kRowUnroll <= count; k += kRowUnroll) {
+      float w[kRowUnroll][8];
+#pragma unroll
+      for (int u = 0; u < kRowUnroll; ++u) load8<T>(weight + (v0 + k + u) * dim + col, w[u]);
+#pragma unroll
+      for (int u = 0; u < kRowUnroll; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(c[k + u], w[u][e], acc[e]);
+    }
+    for (; k < count; ++k) {
+      float w[8];
+      load8<T>(weight + (v0 + k) * dim + col, w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(c[k], w[e], acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) total[e] += acc[e];
+  }
+  float* p = partial + (static_cast<int64_t>(blockIdx.z) * groups + group) * dim + col;
+  *reinterpret_cast<vjp_f32x4*>(p) = vjp_f32x4{total[0], total[1], total[2], total[3]};
+  *reinterpret_cast<vjp_f32x4*>(p + 4) = vjp_f32x4{total[4], total[5], total[6], total[7]};
 }
 
 // grid: (ceil(dim / 64), rows). Thread (group g, column c) sums blocks g, g + 16, ... of column
@@ -404,7 +449,7 @@ __global__ __launch_bounds__(kReduceThreads) void row_sum_reduce_kernel(
     const T* __restrict__ weight, int64_t vocab, const int64_t* __restrict__ targets,
     const float* __restrict__ due, const float* __restrict__ gate, float* __restrict__ out,
     const int64_t* __restrict__ layer_table) {
-  constexpr int kGroups = kReduceThreads / kReduceColumns;
+  constexpr int kGroups = kReduceGroups;
   __shared__ float sums[kGroups][kReduceColumns];
   const int tid = threadIdx.x, g = tid / kReduceColumns, c = tid - g * kReduceColumns;
   if (layer_table) {  // blockIdx.z = layer: its partials, gate and output
@@ -492,11 +537,23 @@ extern "C" int lr_head_logits(const float* hidden, int64_t rows, const void* wei
   if (int status = check_weight(dtype, vocab, dim, weight)) return status;
   LR_REQUIRE(rows > 0 && hidden && out, "Invalid hidden states");
   const hipStream_t s = as_stream(stream);
+  if (rows > 1 && takes_head_products(dtype, vocab, dim) && reinterpret_cast<uintptr_t>(hidden) % 16 == 0) {
+    for (int64_t r0 = 0; r0 < rows; r0 += kProductRows) {
+      const int64_t here = std::min<int64_t>(kProductRows, rows - r0);
+      if (int status = launch_head_products(hidden + r0 * dim, here, weight, bias, vocab, dim,
+                                            out + r0 * vocab, s))
+        return status;
+    }
+    return LR_OK;
+  }
   const int64_t per_pass = std::min<int64_t>(8, kLogitLdsFloats / dim);
-  const int64_t blocks = ceil_div(vocab, kLogitRowsPerBlock);
   for (int64_t r0 = 0; r0 < rows; r0 += per_pass) {
     const int64_t here = std::min<int64_t>(per_pass, rows - r0);
     const int rp = row_pass(here);
+    const int64_t lds = rp * dim * static_cast<int64_t>(sizeof(float));
+    const int64_t resident = 256 * std::min<int64_t>(8, (160 << 10) / lds);
+    int64_t blocks = ceil_div(vocab, kLogitRowsPerBlock);
+    if (rp > 1) blocks = std::min(blocks, resident);
     const int status = dispatch_weight(dtype, [&]<typename T>() {
       const T* w = static_cast<const T*>(weight);
       const T* b = static_cast<const T*>(bias);
@@ -553,7 +610,9 @@ extern "C" int lr_margin_stats(const float* logits, int64_t rows, int64_t vocab,
 extern "C" size_t lr_row_sum_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
   if (rows <= 0 || vocab <= 0 || dim <= 0) return 0;
   const int64_t pass = std::min<int64_t>(rows, 8);
-  const int64_t blocks = ceil_div(vocab, rows_per_block(vocab, dim, row_pass(pass)));
+  int64_t blocks = ceil_div(vocab, rows_per_block(vocab, dim, row_pass(pass)));
+  if (takes_column_products(LR_DTYPE_BF16, pass, dim))  // whichever kernel the weight's type takes
+    blocks = std::max(blocks, ceil_div(vocab, column_product_block_rows(vocab, dim)));
   return static_cast<size_t>(blocks) * static_cast<size_t>(pass) * static_cast<size_t>(dim) *
          sizeof(float);
 }
@@ -570,8 +629,10 @@ int weighted_rows(const void* weight, int dtype, int64_t vocab, int64_t dim, int
   LR_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "Workspace must be 16-byte aligned");
   for (int64_t r0 = 0; r0 < rows; r0 += 8) {
     const int64_t here = std::min<int64_t>(8, rows - r0);
+    const bool products = logits && takes_column_products(dtype, here, dim);
     const int rp = row_pass(here);
-    const int64_t per_block = rows_per_block(vocab, dim, rp);
+    const int64_t per_block =
+        products ? column_product_block_rows(vocab, dim) : rows_per_block(vocab, dim, rp);
     const int64_t blocks = ceil_div(vocab, per_block);
     RowSumArgs args{};
     args.weight = weight;
@@ -587,7 +648,9 @@ int weighted_rows(const void* weight, int dtype, int64_t vocab, int64_t dim, int
     const size_t lds = static_cast<size_t>(per_block) * rp * sizeof(float);
     const dim3 grid(static_cast<unsigned>(ceil_div(dim, kRowSumColumns)),
                     static_cast<unsigned>(blocks));
-    int status = dispatch_weight(dtype, [&]<typename T>() {
+    int status = products ? launch_column_products(weight, vocab, dim, here, args.logits,
+                                                   args.stats, args.targets, args.partial, stream)
+                          : dispatch_weight(dtype, [&]<typename T>() {
       auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kRowSumThreads), lds, stream, args);
         return check_launch("row_sum");
@@ -641,8 +704,8 @@ extern "C" int lr_pre_gradient(const float* post_gradient, const void* o_weight,
 
 extern "C" size_t lr_pre_gradient_layers_workspace_bytes(int64_t layers, int64_t hidden,
                                                          int64_t width) {
-  if (layers <= 0) return 0;
-  return static_cast<size_t>(layers) * lr_row_sum_workspace_bytes(1, hidden, width);
+  if (layers <= 0 || hidden <= 0 || width <= 0) return 0;
+  return static_cast<size_t>(layers) * kReduceGroups * static_cast<size_t>(width) * sizeof(float);
 }
 
 extern "C" int lr_pre_gradient_layers(const int64_t* layer_table, int64_t layers, int64_t hidden,
@@ -661,20 +724,15 @@ extern "C" int lr_pre_gradient_layers(const int64_t* layer_table, int64_t layers
              "Row-sum workspace too small");
   const int64_t per_block = rows_per_block(hidden, width, 1);
   const int64_t blocks = ceil_div(hidden, per_block);
-  RowSumArgs args{};
-  args.vocab = hidden;
-  args.dim = width;
-  args.rows = 1;
-  args.rows_per_block = per_block;
-  args.partial = static_cast<float*>(workspace);
-  args.layer_table = layer_table;
+  const int64_t groups = std::min<int64_t>(blocks, kReduceGroups);
+  float* partial = static_cast<float*>(workspace);
   const hipStream_t s = as_stream(stream);
-  const size_t lds = static_cast<size_t>(per_block) * sizeof(float);
   int status = dispatch_weight(dtype, [&]<typename T>() {
-    hipLaunchKernelGGL((row_sum_kernel<T, 1>),
+    hipLaunchKernelGGL(row_sum_layers_kernel<T>,
                        dim3(static_cast<unsigned>(ceil_div(width, kRowSumColumns)),
-                            static_cast<unsigned>(blocks), static_cast<unsigned>(layers)),
-                       dim3(kRowSumThreads), lds, s, args);
+                            static_cast<unsigned>(groups), static_cast<unsigned>(layers)),
+                       dim3(kRowSumThreads), 0, s, layer_table, hidden, width, per_block, blocks,
+                       partial);
     return check_launch("row_sum");
   });
   if (status) return status;
@@ -682,7 +740,7 @@ extern "C" int lr_pre_gradient_layers(const int64_t* layer_table, int64_t layers
     hipLaunchKernelGGL(row_sum_reduce_kernel<T>,
                        dim3(static_cast<unsigned>(ceil_div(width, kReduceColumns)), 1u,
                             static_cast<unsigned>(layers)),
-                       dim3(kReduceThreads), 0, s, static_cast<const float*>(workspace), blocks,
+                       dim3(kReduceThreads), 0, s, static_cast<const float*>(partial), groups,
                        int64_t{1}, width, static_cast<const T*>(nullptr), hidden, nullptr,
                        nullptr, nullptr, nullptr, layer_table);
     return check_launch("row_sum_reduce");

@@ -45,6 +45,67 @@ def test_head_logits(device, dtype, rows, vocab, dim, bias):
     assert np.all(np.abs(got - expect) <= 1e-5 * scale + 1e-6)
 
 
+@pytest.mark.parametrize("rows,vocab,dim,bias", [
+    (2, 32, 1024, False),    # one weight tile, one stage a wave
+    (8, 33, 2048, True),     # a last tile that reaches back over the first
+    (9, 8193, 3072, False),  # two row passes (the second of one row), a ragged last tile
+    (5, 97, 5120, True),     # the largest hidden size of the matrix-core kernel
+    (4, 31, 1024, True),     # fewer weight rows than a tile
+    (6, 300, 1536, False),   # a hidden size the matrix-core kernel does not take
+])
+def test_head_logits_several_rows(device, rows, vocab, dim, bias):
+    """Several f32 rows (all 24 significant bits) against a bf16 weight, from a buffer that is
+    16-byte aligned and from one that is not: both kernels' row, tile and stage edges."""
+    model, weight = model_with_head(device, vocab, dim, bias=bias, seed=rows + 30)
+    x = torch.randn((rows, dim), generator=torch.Generator().manual_seed(31)) * 3
+    b = None if not bias else model.get_output_embeddings().bias.double().cpu().numpy()
+    expect = ovjp.head_logits(x.double().numpy(), weight, b)
+    scale = np.abs(x.double().numpy()) @ np.abs(weight).T + (0 if b is None else np.abs(b))
+    shifted = torch.empty(rows * dim + 1, device=device)[1:].view(rows, dim)
+    assert shifted.data_ptr() % 16 == 4
+    for hidden in (x.to(device), shifted.copy_(x)):
+        got = vjp.last_token_logits_float32(model, hidden).cpu().numpy()
+        # the longest f32 chain is 128 sums a row part and eight parts: well under 1e-6 of scale
+        assert np.all(np.abs(got - expect) <= 1e-6 * scale)
+
+
+def test_head_logits_non_finite_rows_and_weights(device):
+    """Infinities and NaN go where f32 arithmetic takes them, and nowhere else."""
+    model, weight = model_with_head(device, 64, 1024, seed=40)
+    x = torch.randn((3, 1024), generator=torch.Generator().manual_seed(41))
+    x[0, 5], x[1, 900] = float("inf"), float("nan")
+    clean = vjp.last_token_logits_float32(model, x[2:].repeat(2, 1).to(device))[:1]
+    got = vjp.last_token_logits_float32(model, x.to(device)).cpu()
+    signs = torch.from_numpy(np.sign(weight[:, 5])).float()
+    assert torch.equal(got[0], signs * float("inf")) and torch.isnan(got[1]).all()
+    assert torch.equal(got[2], clean[0].cpu())
+    w = model.get_output_embeddings().weight
+    w[7, 3] = float("-inf")
+    x[2, 3] = 2.0  # its second and third pieces are zero
+    got = vjp.last_token_logits_float32(model, x.to(device)).cpu()
+    assert got[2, 7] == float("-inf") and torch.isfinite(got[2][torch.arange(64) != 7]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,vocab,dim", [(3, 17, 128), (8, 513, 640), (5, 4100, 512),
+                                            (11, 1000, 1024), (8, 200, 1000)])
+def test_row_hidden_gradients_several_rows(device, dtype, rows, vocab, dim):
+    """Ragged weight rows and column blocks, two row passes (8 and 3), and a width that the
+    matrix-core kernel does not take (1000)."""
+    model, weight = model_with_head(device, vocab, dim, dtype, seed=rows + 50)
+    logits = torch.randn((rows, vocab), generator=torch.Generator().manual_seed(51)).to(device) * 3
+    _, targets, competitors = vjp.row_margins(logits)
+    due = [float(r != 1) for r in range(rows)]
+    got = vjp.row_hidden_gradients(model, logits, targets, competitors, due).cpu().numpy()
+    l64, t = logits.double().cpu().numpy(), targets.cpu().numpy()
+    expect = ovjp.hidden_gradient(l64, t, weight, np.array(due))
+    share = np.exp(l64 - l64.max(axis=1, keepdims=True))
+    share[np.arange(rows), t] = 0
+    scale = np.abs(weight[t]) + (share / share.sum(axis=1, keepdims=True)) @ np.abs(weight)
+    # the shares carry expf's and the division's f32 rounding, the sums chains of at most 32 + 251
+    assert np.all(np.abs(got - expect) <= 2e-6 * scale)
+
+
 def test_margins_given_and_argmax(device):
     rng = np.random.default_rng(3)
     logits = (rng.standard_normal((4, 128256)) * 3).astype(np.float32)
