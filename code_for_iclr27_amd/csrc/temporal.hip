@@ -15,9 +15,6 @@
 namespace lr {
 namespace {
 
-constexpr int kRowThreads = 256;
-constexpr int kWaves = kRowThreads / 64;
-
 template <bool kMax>
 __device__ __forceinline__ float wave_reduce(float v) {
 #pragma unroll
@@ -28,8 +25,9 @@ __device__ __forceinline__ float wave_reduce(float v) {
   return v;
 }
 
-// Block-wide reduction for 256 threads; every thread receives the result.
-template <bool kMax>
+// Block-wide reduction over WAVES waves; every thread receives the result. `scratch` holds one
+// value a wave and is used once (no barrier before its reuse).
+template <bool kMax, int WAVES>
 __device__ __forceinline__ float block_reduce(float v, float* scratch) {
   v = wave_reduce<kMax>(v);
   const int wave = threadIdx.x >> 6;
@@ -37,8 +35,7 @@ __device__ __forceinline__ float block_reduce(float v, float* scratch) {
   __syncthreads();
   float r = scratch[0];
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) r = kMax ? fmaxf(r, scratch[w]) : r + scratch[w];
-  __syncthreads();
+  for (int w = 1; w < WAVES; ++w) r = kMax ? fmaxf(r, scratch[w]) : r + scratch[w];
   return r;
 }
 
@@ -70,17 +67,22 @@ __device__ __forceinline__ float load_as_float<__bf16>(const __bf16* p, int64_t 
   return static_cast<float>(p[i]);
 }
 
-// One 256-thread block per (query, group) row. Thread t owns positions t, t+256, ...; when a
-// row fits in kCache per-thread registers the masked logits stay in registers across the
-// three phases (max, exp-sum, normalise+project), otherwise they are re-derived from the
-// logits (never from the output buffer).
-template <typename T, int kCache>
-__global__ __launch_bounds__(kRowThreads) void probabilities_kernel(
+// One block per (query, group) row. Thread t owns positions t, t + THREADS, ...: CACHE of them in
+// registers (the masked logits, then the exponentials), so a row is read once. A row is short work
+// (a 8B head: 9 positions a thread), so its time is its chain of memory and barrier latencies:
+// every load of the row, the projected values included, is issued before the first is used
+// (clamped to the row; a load under the bounds check would be waited for inside it). Measured (64
+// queries x 4 groups, calls back to back, us, against 256 threads a row and loads in bounded
+// loops): 2,250 keys 4.7 against 6.3, 16,000 10.8 against 41.6, 33,792 30 against 94.
+// CACHE = 0: longer rows, the masked logits read again in each of the three phases.
+template <typename T, int THREADS, int CACHE>
+__global__ __launch_bounds__(THREADS) void probabilities_kernel(
     const T* __restrict__ logits, const float* __restrict__ projected,
     const int64_t* __restrict__ query_positions, const float* __restrict__ key_positions,
     float* __restrict__ probabilities, float* __restrict__ output_projection, int64_t groups,
     int64_t length, float scale) {
-  __shared__ float scratch[kWaves];
+  constexpr int WAVES = THREADS / 64;
+  __shared__ float scratch[3][WAVES];
   const int64_t row = blockIdx.x;
   const int64_t group = row % groups;
   const int64_t query = row / groups;
@@ -88,39 +90,71 @@ __global__ __launch_bounds__(kRowThreads) void probabilities_kernel(
   const T* in = logits + row * length;
   float* out = probabilities + row * length;
   const float* pv = projected + group * length;
+  const int64_t first = threadIdx.x;
   // Reference compares float key positions against the int64 query position promoted
   // to float (csrc/scoring.cu:46).
-  auto masked = [&](int64_t t) -> float {
-    const float rounded = round_to<T>(load_as_float<T>(in, t) * scale);
-    return key_positions[t] <= query_position ? rounded : -INFINITY;
+  auto masked = [&](float logit, float key_position) -> float {
+    const float rounded = round_to<T>(logit * scale);
+    return key_position <= query_position ? rounded : -INFINITY;
   };
-  float cache[kCache > 0 ? kCache : 1];
-  float maximum = -INFINITY;
-  int i = 0;
-  for (int64_t t = threadIdx.x; t < length; t += kRowThreads, ++i) {
-    const float v = masked(t);
-    if (kCache > 0) cache[i] = v;
-    maximum = fmaxf(maximum, v);
+  float maximum = -INFINITY, denominator = 0.0f, projection = 0.0f;
+  if constexpr (CACHE > 0) {
+    float x[CACHE], k[CACHE], v[CACHE];
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+      const int64_t at = first + i * THREADS < length ? first + i * THREADS : length - 1;
+      x[i] = load_as_float<T>(in, at);
+      k[i] = key_positions[at];
+      v[i] = pv[at];
+    }
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+      x[i] = first + i * THREADS < length ? masked(x[i], k[i]) : -INFINITY;
+      maximum = fmaxf(maximum, x[i]);
+    }
+    maximum = block_reduce<true, WAVES>(maximum, scratch[0]);
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+      if (first + i * THREADS >= length) break;
+      x[i] = expf(x[i] - maximum);
+      denominator += x[i];
+    }
+    denominator = block_reduce<false, WAVES>(denominator, scratch[1]);
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+      if (first + i * THREADS >= length) break;
+      const float p = x[i] / denominator;
+      out[first + i * THREADS] = p;
+      projection += p * v[i];
+    }
+  } else {
+    constexpr int U = 8;  // positions whose loads are in flight together
+    auto visit = [&](auto&& use) {
+      for (int64_t base = first; base < length; base += U * THREADS) {
+        float x[U], k[U], v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const int64_t at = base + i * THREADS < length ? base + i * THREADS : length - 1;
+          x[i] = load_as_float<T>(in, at);
+          k[i] = key_positions[at];
+          v[i] = pv[at];
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+          if (base + i * THREADS < length) use(base + i * THREADS, masked(x[i], k[i]), v[i]);
+      }
+    };
+    visit([&](int64_t, float z, float) { maximum = fmaxf(maximum, z); });
+    maximum = block_reduce<true, WAVES>(maximum, scratch[0]);
+    visit([&](int64_t, float z, float) { denominator += expf(z - maximum); });
+    denominator = block_reduce<false, WAVES>(denominator, scratch[1]);
+    visit([&](int64_t at, float z, float value) {
+      const float p = expf(z - maximum) / denominator;
+      out[at] = p;
+      projection += p * value;
+    });
   }
-  maximum = block_reduce<true>(maximum, scratch);
-  float denominator = 0.0f;
-  i = 0;
-  for (int64_t t = threadIdx.x; t < length; t += kRowThreads, ++i) {
-    const float v = kCache > 0 ? cache[i] : masked(t);
-    const float w = expf(v - maximum);
-    if (kCache > 0) cache[i] = w;
-    denominator += w;
-  }
-  denominator = block_reduce<false>(denominator, scratch);
-  float projection = 0.0f;
-  i = 0;
-  for (int64_t t = threadIdx.x; t < length; t += kRowThreads, ++i) {
-    const float w = kCache > 0 ? cache[i] : expf(masked(t) - maximum);
-    const float p = w / denominator;
-    out[t] = p;
-    projection += p * pv[t];
-  }
-  projection = block_reduce<false>(projection, scratch);
+  projection = block_reduce<false, WAVES>(projection, scratch[2]);
   if (threadIdx.x == 0) output_projection[row] = projection;
 }
 
@@ -132,62 +166,101 @@ __device__ __forceinline__ double risk64(double margin, double probability, doub
   return fmax(0.0, probability * (margin - compared) - base_softplus + softplus64(compared));
 }
 
-// 64 candidate lanes x 4 query lanes per block. Query lane q visits queries q, q+4, ...; the
-// margin drop of one (query, candidate) sums the groups in order g = 0..G-1 exactly like the
-// reference. Any non-finite drop makes the candidate's score NaN.
+// A block of 16 waves takes 64 candidates (one a lane); wave w visits queries w, w + 16, ..., four
+// at a time with every group's probability loaded before the first is used. The margin drop of one
+// (query, candidate) sums the groups in order g = 0..G-1 exactly like the reference. Any
+// non-finite drop makes the candidate's score NaN. There are only as many blocks as 64-candidate
+// columns (35 for an 8B head), so the depth of a wave's loads sets the time: 16 waves of four
+// queries take 5.4 us for 64 queries x 4 groups x 2,218 candidates, four waves one query at a time
+// took 14.5 (calls back to back).
 constexpr int kRiskCandidates = 64;
-constexpr int kRiskQueryLanes = 4;
+constexpr int kRiskWaves = 16;
+constexpr int kRiskQueries = 4;
 
-__global__ __launch_bounds__(kRiskCandidates* kRiskQueryLanes) void risk_kernel(
+// GROUPS: the group count known at compile time (loads of all groups in flight), or 0.
+template <int GROUPS>
+__global__ __launch_bounds__(kRiskCandidates* kRiskWaves) void risk_kernel(
     const float* __restrict__ probabilities, const float* __restrict__ output_projection,
     const float* __restrict__ projected, const float* __restrict__ margin,
-    float* __restrict__ result, int64_t window, int64_t groups, int64_t length, int64_t first,
+    float* __restrict__ result, int64_t window, int64_t groups_in, int64_t length, int64_t first,
     int64_t count, float epsilon) {
-  __shared__ float minimums[kRiskQueryLanes][kRiskCandidates];
-  __shared__ float maximums[kRiskQueryLanes][kRiskCandidates];
-  __shared__ int bad[kRiskQueryLanes][kRiskCandidates];
+  __shared__ float minimums[kRiskWaves][kRiskCandidates];
+  __shared__ float maximums[kRiskWaves][kRiskCandidates];
+  __shared__ int bad[kRiskWaves][kRiskCandidates];
+  __shared__ double terms[2];
+  __shared__ double upper_risk[kRiskCandidates];
+  const int64_t groups = GROUPS ? GROUPS : groups_in;
   const int lane = threadIdx.x % kRiskCandidates;
-  const int query_lane = threadIdx.x / kRiskCandidates;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kRiskCandidates);
   const int64_t candidate = static_cast<int64_t>(blockIdx.x) * kRiskCandidates + lane;
-  const int64_t position = first + candidate;
+  const bool live = candidate < count;
+  const int64_t position = first + (live ? candidate : count - 1);
   float minimum = INFINITY, maximum = -INFINITY;
   int nonfinite = 0;
-  if (candidate < count) {
-    for (int64_t query = query_lane; query < window; query += kRiskQueryLanes) {
+  auto drop_term = [&](float p, float value, float output) {
+    const float ratio = p / fmaxf(1.0f - p, epsilon);
+    return ratio * (value - output);
+  };
+  auto visit = [&](float drop) {
+    if (!isfinite(drop)) nonfinite = 1;
+    minimum = fminf(minimum, drop);
+    maximum = fmaxf(maximum, drop);
+  };
+  if constexpr (GROUPS > 0) {
+    float value[GROUPS];
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) value[g] = projected[g * length + position];
+    for (int64_t q0 = wave; q0 < window; q0 += kRiskWaves * kRiskQueries) {
+      float p[kRiskQueries][GROUPS];
+#pragma unroll
+      for (int j = 0; j < kRiskQueries; ++j) {
+        const int64_t q = q0 + j * kRiskWaves < window ? q0 + j * kRiskWaves : q0;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) p[j][g] = probabilities[(q * GROUPS + g) * length + position];
+      }
+#pragma unroll
+      for (int j = 0; j < kRiskQueries; ++j) {
+        const int64_t q = q0 + j * kRiskWaves;
+        if (q >= window) break;
+        float drop = 0.0f;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+          drop += drop_term(p[j][g], value[g], output_projection[q * GROUPS + g]);
+        visit(drop);
+      }
+    }
+  } else {
+    for (int64_t q = wave; q < window; q += kRiskWaves) {
       float drop = 0.0f;
-      for (int64_t group = 0; group < groups; ++group) {
-        const int64_t row = query * groups + group;
-        const float p = probabilities[row * length + position];
-        const float ratio = p / fmaxf(1.0f - p, epsilon);
-        drop += ratio * (projected[group * length + position] - output_projection[row]);
-      }
-      if (!isfinite(drop)) {
-        nonfinite = 1;
-        break;
-      }
-      minimum = fminf(minimum, drop);
-      maximum = fmaxf(maximum, drop);
+      for (int64_t g = 0; g < groups; ++g)
+        drop += drop_term(probabilities[(q * groups + g) * length + position],
+                          projected[g * length + position], output_projection[q * groups + g]);
+      visit(drop);
     }
   }
-  minimums[query_lane][lane] = minimum;
-  maximums[query_lane][lane] = maximum;
-  bad[query_lane][lane] = nonfinite;
+  minimums[wave][lane] = minimum;
+  maximums[wave][lane] = maximum;
+  bad[wave][lane] = nonfinite;
+  const double m = static_cast<double>(margin[0]);
+  if (threadIdx.x == kRiskCandidates * (kRiskWaves - 1)) {  // the margin's terms, once
+    terms[0] = 1.0 / (1.0 + exp(-m));
+    terms[1] = softplus64(m);
+  }
   __syncthreads();
-  if (query_lane == 0 && candidate < count) {
-    for (int q = 1; q < kRiskQueryLanes; ++q) {
-      minimum = fminf(minimum, minimums[q][lane]);
-      maximum = fmaxf(maximum, maximums[q][lane]);
-      nonfinite |= bad[q][lane];
+  // Wave 0 takes the risk of the minimum, wave 1 that of the maximum.
+  double risk = 0.0;
+  if (wave < 2) {
+    for (int w = 0; w < kRiskWaves; ++w) {
+      minimum = fminf(minimum, minimums[w][lane]);
+      maximum = fmaxf(maximum, maximums[w][lane]);
+      nonfinite |= bad[w][lane];
     }
-    if (nonfinite) {
-      result[candidate] = NAN;
-      return;
-    }
-    const double m = static_cast<double>(margin[0]);
-    const double p = 1.0 / (1.0 + exp(-m));
-    const double base = softplus64(m);
-    result[candidate] = static_cast<float>(fmax(risk64(m, p, base, minimum), risk64(m, p, base, maximum)));
+    risk = risk64(m, terms[0], terms[1], wave ? maximum : minimum);
+    if (wave) upper_risk[lane] = risk;
   }
+  __syncthreads();
+  if (wave == 0 && live)
+    result[candidate] = nonfinite ? NAN : static_cast<float>(fmax(risk, upper_risk[lane]));
 }
 
 // Sliding max of odd width inside each segment; NaN neighbours are ignored as by fmaxf and
@@ -292,13 +365,16 @@ int launch_probabilities(const void* logits, const float* projected, const int64
                          hipStream_t stream) {
   const int64_t rows = window * groups;
   const T* in = static_cast<const T*>(logits);
-  if (length <= 256 * 16) {
-    probabilities_kernel<T, 16><<<rows, kRowThreads, 0, stream>>>(
+  auto launch = [&](auto kernel, int threads) {
+    kernel<<<static_cast<unsigned>(rows), threads, 0, stream>>>(
         in, projected, qpos, kpos, probabilities, output_projection, groups, length, scale);
-  } else {
-    probabilities_kernel<T, 0><<<rows, kRowThreads, 0, stream>>>(
-        in, projected, qpos, kpos, probabilities, output_projection, groups, length, scale);
-  }
+  };
+  // The smallest cache that holds the row: unused positions cost loads of the row's last one.
+  if (length <= 256 * 4) launch(probabilities_kernel<T, 256, 4>, 256);
+  else if (length <= 256 * 9) launch(probabilities_kernel<T, 256, 9>, 256);
+  else if (length <= 256 * 16) launch(probabilities_kernel<T, 256, 16>, 256);
+  else if (length <= 1024 * 16) launch(probabilities_kernel<T, 1024, 16>, 1024);
+  else launch(probabilities_kernel<T, 1024, 0>, 1024);
   return check_launch("temporal_probabilities");
 }
 
@@ -349,9 +425,21 @@ extern "C" int lr_temporal_risk(const float* probabilities, const float* output_
              "Expected contiguous CUDA tensor");
   const int64_t count = last - first;
   const int64_t blocks = ceil_div(count, kRiskCandidates);
-  risk_kernel<<<blocks, kRiskCandidates * kRiskQueryLanes, 0, as_stream(stream)>>>(
-      probabilities, output_projection, projected, margin, result, window, groups, length, first,
-      count, static_cast<float>(epsilon));
+  const hipStream_t s = as_stream(stream);
+  const float eps = static_cast<float>(epsilon);
+  auto launch = [&](auto kernel) {
+    kernel<<<static_cast<unsigned>(blocks), kRiskCandidates * kRiskWaves, 0, s>>>(
+        probabilities, output_projection, projected, margin, result, window, groups, length, first,
+        count, eps);
+  };
+  switch (groups) {
+    case 1: launch(risk_kernel<1>); break;
+    case 2: launch(risk_kernel<2>); break;
+    case 4: launch(risk_kernel<4>); break;
+    case 6: launch(risk_kernel<6>); break;
+    case 8: launch(risk_kernel<8>); break;
+    default: launch(risk_kernel<0>); break;
+  }
   return check_launch("temporal_risk");
 }
 

@@ -65,6 +65,34 @@ def test_temporal_risk(device, shape, first, last):
     np.testing.assert_allclose(to_np(got), expect, rtol=1e-5, atol=1e-12)
 
 
+@pytest.mark.parametrize("window,groups,length,first,last", [
+    (1, 1, 1, 0, 1), (15, 2, 64, 0, 64), (16, 3, 1024, 1, 65), (17, 4, 1025, 0, 993),
+    (63, 5, 2304, 5, 70), (64, 6, 2305, 0, 2273), (65, 7, 4096, 4000, 4096),
+    (129, 8, 4097, 17, 4065), (9, 4, 16384, 16000, 16384), (5, 2, 16385, 0, 640),
+    (3, 1, 40000, 39000, 39999)])
+def test_temporal_ops_across_row_and_window_sizes(device, window, groups, length, first, last):
+    """Every way the rows are held (4, 9 or 16 positions a thread, wide blocks, re-read rows) and
+    the risk's queries are shared out (whole and partial rounds of waves, group counts with and
+    without their own kernel), with a query that sees no key."""
+    shape = (window, groups, length)
+    logits = rand(shape, torch.bfloat16, device, 11, scale=math.sqrt(128))
+    pv = rand((groups, length), torch.float32, device, 12, scale=10)
+    qpos = torch.arange(length - window, length, device=device)
+    kpos = torch.arange(length, device=device).float()
+    scale = 1.0 / math.sqrt(128)
+    p, op = _C.temporal_probabilities(logits, pv, qpos, kpos, scale)
+    ep, eop = oscoring.temporal_probabilities(to_np(logits), to_np(pv), qpos.cpu().numpy(),
+                                              kpos.cpu().numpy(), np.float32(scale), "bf16")
+    np.testing.assert_allclose(to_np(p), ep, rtol=1e-5, atol=1e-30)
+    np.testing.assert_allclose(to_np(op), eop, rtol=1e-5, atol=1e-5)
+    margin = torch.tensor([2.0], device=device)
+    got = _C.temporal_risk(p, op, pv, margin, first, last, 1e-6)
+    expect = oscoring.temporal_risk(to_np(p), to_np(op), to_np(pv), np.float32(2.0), first, last, 1e-6)
+    np.testing.assert_allclose(to_np(got), expect, rtol=1e-5, atol=1e-12)
+    blind, _ = _C.temporal_probabilities(logits, pv, torch.full_like(qpos, -1), kpos, scale)
+    assert torch.isnan(blind).all()  # exp(-inf - -inf), as the definition has it
+
+
 def test_temporal_risk_nonfinite(device):
     p = torch.full((3, 2, 10), 0.1, device=device)
     op = torch.zeros((3, 2), device=device)
