@@ -38,6 +38,7 @@ SIGNATURES = {
     "lr_abi_version": [],
     "lr_temporal_probabilities": [_P, _I, _P, _P, _P, _I64, _I64, _I64, _F, _P, _P, _P],
     "lr_temporal_risk": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _D, _P, _P],
+    "lr_temporal_risk_max": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _D, _P, _P],
     "lr_append": [_P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I, _I64, _I64, _P, _P, _P, _P,
                   _P, _P],
     "lr_append_layers": [_P, _I64, _I64, _I64, _I64, _I, _I64, _P, _P, _P, _P, _P, _P],

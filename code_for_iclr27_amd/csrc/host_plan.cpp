@@ -231,6 +231,9 @@ struct Library {
   decltype(&lr_queue_index) queue_index = nullptr;
   decltype(&lr_queue_evict_plan) queue_evict_plan = nullptr;
   decltype(&lr_compact_heads_layout) compact_heads = nullptr;
+  decltype(&lr_temporal_probabilities) temporal_probabilities = nullptr;
+  decltype(&lr_temporal_risk) temporal_risk = nullptr;
+  decltype(&lr_temporal_risk_max) temporal_risk_max = nullptr;
   decltype(&lr_append) append = nullptr;
   decltype(&lr_compact) compact = nullptr;
   decltype(&lr_append_layers) append_layers = nullptr;
@@ -276,6 +279,13 @@ void bind_library(int64_t score_workspace_bytes, int64_t score_segments, int64_t
   bind_one(library.staging_alloc, staging_alloc);
   bind_one(library.staging_free, staging_free);
   bind_one(library.copy_words, copy_words);
+}
+
+void bind_temporal(int64_t probabilities, int64_t risk, int64_t risk_max, int64_t last_error) {
+  bind_one(library.temporal_probabilities, probabilities);
+  bind_one(library.temporal_risk, risk);
+  bind_one(library.temporal_risk_max, risk_max);
+  bind_one(library.last_error, last_error);
 }
 
 void bind_data_movement(int64_t append, int64_t compact, int64_t append_layers,
@@ -1640,6 +1650,68 @@ std::vector<torch::Tensor> batch_append_launch(const std::vector<torch::Tensor>&
   return {out_keys, out_values, out_positions};
 }
 
+// ---------------------------------------------------------------------------------------
+// scoring.temporal_head_scores on the device: the per-chunk loop of scoring.py:177-194 (logits by
+// torch's product, temporal_probabilities, temporal_risk, the maximum over chunks) with the
+// checks the operators make. A head is about 85 us of device work in small launches; made from
+// Python it took 240 us, bound by the host, from here 133 (8B shape, four chunks). The chunks share one probabilities
+// buffer, and a chunk's scores are folded into the first one's by the risk kernel.
+// The arguments were checked by the caller as far as they are Python's to check.
+torch::Tensor temporal_head_scores(const torch::Tensor& queries, const torch::Tensor& query_positions_in,
+                                   const torch::Tensor& keys, const torch::Tensor& key_positions_in,
+                                   const torch::Tensor& values, int64_t first, int64_t last,
+                                   const torch::Tensor& gradient, const torch::Tensor& margin_in,
+                                   double epsilon, int64_t chunk) {
+  require(library.temporal_risk_max != nullptr, "library entry points are not bound");
+  const torch::Device device = keys.device();
+  const at::NoGradGuard no_grad;
+  const torch::Tensor projected =
+      at::matmul(gradient.to(torch::kFloat32), values.to(torch::kFloat32).transpose(0, 1)).contiguous();
+  const torch::Tensor key_positions = key_positions_in.to(torch::kFloat32).contiguous();
+  const torch::Tensor query_positions = query_positions_in.to(torch::kInt64).contiguous();
+  const torch::Tensor margin =
+      margin_in.to(torch::TensorOptions().device(device).dtype(torch::kFloat32)).reshape({1}).contiguous();
+  for (const torch::Tensor* t : {&projected, &query_positions, &key_positions}) {
+    require(t->is_cuda(), "Expected contiguous CUDA tensor");
+    require(t->device() == device, "CUDA devices differ");
+  }
+  const int64_t window = queries.size(0), groups = queries.size(1), dim = queries.size(2);
+  const int64_t length = keys.size(0);
+  require(groups > 0, "Empty attention dimensions");
+  require(projected.dim() == 2 && projected.size(0) == groups && projected.size(1) == length,
+          "Invalid projected values");
+  require(query_positions.numel() == window, "Invalid query positions");
+  require(key_positions.numel() == length, "Invalid key positions");
+  const c10::DeviceGuard guard(device);
+  const auto f32 = keys.options().dtype(torch::kFloat32).requires_grad(false);
+  const int64_t most = std::min(chunk, window);
+  const torch::Tensor probabilities = torch::empty({most, groups, length}, f32);
+  const torch::Tensor output = torch::empty({most, groups}, f32);
+  torch::Tensor result = torch::empty({last - first}, f32);
+  const torch::Tensor keys_t = keys.transpose(0, 1);
+  const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(dim)));
+  void* stream = current_stream(device);
+  for (int64_t start = 0; start < window; start += chunk) {
+    const int64_t here = std::min(chunk, window - start);
+    const torch::Tensor logits =
+        at::matmul(queries.narrow(0, start, here).to(keys.scalar_type()), keys_t).contiguous();
+    const auto dtype = logits.scalar_type();
+    require(dtype == torch::kFloat32 || dtype == torch::kHalf || dtype == torch::kBFloat16,
+            "Only FP32/FP16/BF16 scores are supported");
+    check_call(library.temporal_probabilities(
+        logits.data_ptr(),
+        dtype == torch::kFloat32 ? LR_DTYPE_F32 : dtype == torch::kHalf ? LR_DTYPE_F16 : LR_DTYPE_BF16,
+        projected.data_ptr<float>(),
+        query_positions.data_ptr<int64_t>() + start, key_positions.data_ptr<float>(), here, groups,
+        length, scale, probabilities.data_ptr<float>(), output.data_ptr<float>(), stream));
+    check_call((start ? library.temporal_risk_max : library.temporal_risk)(
+        probabilities.data_ptr<float>(), output.data_ptr<float>(), projected.data_ptr<float>(),
+        margin.data_ptr<float>(), here, groups, length, first, last, epsilon,
+        result.data_ptr<float>(), stream));
+  }
+  return result;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_plan, module) {
@@ -1647,6 +1719,9 @@ PYBIND11_MODULE(_plan, module) {
   module.def("bind_library", &bind_library, "Bind the entry points of liblazyrecall_hip.so");
   module.def("bind_data_movement", &bind_data_movement,
              "Bind lr_append and lr_compact of liblazyrecall_hip.so");
+  module.def("bind_temporal", &bind_temporal, "Bind the temporal operators");
+  module.def("temporal_head_scores", &temporal_head_scores,
+             "scoring.temporal_head_scores (src/lazy_recall/scoring.py:171-195), whole");
   module.def("append", &append_launch, "_C.append (csrc/scoring.cu:264-292)");
   module.def("compact", &compact_launch, "_C.compact (csrc/scoring.cu:294-314)");
   module.def("append_layers", &append_layers_launch, "One decode step's append into every layer");

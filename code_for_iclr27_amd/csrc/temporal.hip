@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kRiskCandidates* kRiskWaves) void risk_kernel(
     const float* __restrict__ probabilities, const float* __restrict__ output_projection,
     const float* __restrict__ projected, const float* __restrict__ margin,
     float* __restrict__ result, int64_t window, int64_t groups_in, int64_t length, int64_t first,
-    int64_t count, float epsilon) {
+    int64_t count, float epsilon, int accumulate) {
   __shared__ float minimums[kRiskWaves][kRiskCandidates];
   __shared__ float maximums[kRiskWaves][kRiskCandidates];
   __shared__ int bad[kRiskWaves][kRiskCandidates];
@@ -259,8 +259,11 @@ __global__ __launch_bounds__(kRiskCandidates* kRiskWaves) void risk_kernel(
     if (wave) upper_risk[lane] = risk;
   }
   __syncthreads();
-  if (wave == 0 && live)
-    result[candidate] = nonfinite ? NAN : static_cast<float>(fmax(risk, upper_risk[lane]));
+  if (wave == 0 && live) {
+    float score = nonfinite ? NAN : static_cast<float>(fmax(risk, upper_risk[lane]));
+    if (accumulate) score = __builtin_elementwise_maximum(score, result[candidate]);
+    result[candidate] = score;
+  }
 }
 
 // Sliding max of odd width inside each segment; NaN neighbours are ignored as by fmaxf and
@@ -413,11 +416,12 @@ extern "C" int lr_temporal_probabilities(const void* logits, int logits_dtype,
   }
 }
 
-extern "C" int lr_temporal_risk(const float* probabilities, const float* output_projection,
-                                const float* projected, const float* margin, int64_t window,
-                                int64_t groups, int64_t length, int64_t first, int64_t last,
-                                double epsilon, float* result, void* stream) {
-  clear_error();
+namespace lr {
+namespace {
+
+int risk_scores(const float* probabilities, const float* output_projection, const float* projected,
+                const float* margin, int64_t window, int64_t groups, int64_t length, int64_t first,
+                int64_t last, double epsilon, float* result, int accumulate, void* stream) {
   LR_REQUIRE(window > 0 && groups > 0 && first >= 0 && last > first && last <= length &&
                  epsilon > 0,
              "Invalid risk interval");
@@ -430,7 +434,7 @@ extern "C" int lr_temporal_risk(const float* probabilities, const float* output_
   auto launch = [&](auto kernel) {
     kernel<<<static_cast<unsigned>(blocks), kRiskCandidates * kRiskWaves, 0, s>>>(
         probabilities, output_projection, projected, margin, result, window, groups, length, first,
-        count, eps);
+        count, eps, accumulate);
   };
   switch (groups) {
     case 1: launch(risk_kernel<1>); break;
@@ -441,6 +445,27 @@ extern "C" int lr_temporal_risk(const float* probabilities, const float* output_
     default: launch(risk_kernel<0>); break;
   }
   return check_launch("temporal_risk");
+}
+
+}  // namespace
+}  // namespace lr
+
+extern "C" int lr_temporal_risk(const float* probabilities, const float* output_projection,
+                                const float* projected, const float* margin, int64_t window,
+                                int64_t groups, int64_t length, int64_t first, int64_t last,
+                                double epsilon, float* result, void* stream) {
+  clear_error();
+  return risk_scores(probabilities, output_projection, projected, margin, window, groups, length,
+                     first, last, epsilon, result, 0, stream);
+}
+
+extern "C" int lr_temporal_risk_max(const float* probabilities, const float* output_projection,
+                                    const float* projected, const float* margin, int64_t window,
+                                    int64_t groups, int64_t length, int64_t first, int64_t last,
+                                    double epsilon, float* result, void* stream) {
+  clear_error();
+  return risk_scores(probabilities, output_projection, projected, margin, window, groups, length,
+                     first, last, epsilon, result, 1, stream);
 }
 
 namespace lr {

@@ -3,7 +3,7 @@
 Two entry points:
 
 * ``temporal_head_scores`` — the reference's GPU host path for one KV head
-  (src/lazy_recall/scoring.py:152-195), calling this package's ``_C.temporal_probabilities``
+  (src/lazy_recall/scoring.py:152-195), launching the kernels of ``_C.temporal_probabilities``
   and ``_C.temporal_risk`` exactly where the reference calls ``lazy_recall._C``.
 * ``compute_score_table`` — the same scores for every (layer, KV head) of an audit in one
   fused launch sequence (``lr_score_segments``), replacing the reference's per-head Python
@@ -21,7 +21,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
-from . import _C, _lib
+from . import _lib
 
 
 @dataclass(frozen=True)
@@ -61,7 +61,8 @@ class LayerState:
 def temporal_head_scores(queries, query_positions, keys, key_positions, values, candidate_start,
                          candidate_end, margin_gradient, base_margin, denominator_epsilon,
                          query_chunk_size):
-    """scoring.py:152-195 (GPU branch) with this package's ``_C`` ops."""
+    """scoring.py:152-195 (GPU branch) with this package's operators, in C++ after these checks
+    (csrc/host_plan.cpp temporal_head_scores)."""
     if not keys.is_cuda:
         raise RuntimeError("temporal_head_scores requires CUDA tensors (no CPU fallback)")
     if queries.ndim != 3 or queries.shape[-1] != keys.shape[-1]:
@@ -74,23 +75,28 @@ def temporal_head_scores(queries, query_positions, keys, key_positions, values, 
         raise ValueError("Invalid candidate interval")
     if query_chunk_size <= 0 or denominator_epsilon <= 0:
         raise ValueError("Chunk size and denominator epsilon must be positive")
-    projected = torch.matmul(margin_gradient.float(), values.float().transpose(0, 1)).contiguous()
-    key_positions = key_positions.to(dtype=torch.float32).contiguous()
-    query_positions = query_positions.to(dtype=torch.int64).contiguous()
-    margin = base_margin.to(device=keys.device, dtype=torch.float32).reshape(1).contiguous()
     bytes_per_query = queries.shape[1] * keys.shape[0] * (keys.element_size() + 4)
     chunk = min(query_chunk_size, max(1, (64 * 1024 ** 2) // bytes_per_query))
-    result = None
-    for start in range(0, queries.shape[0], chunk):
-        end = min(start + chunk, queries.shape[0])
-        logits = torch.matmul(queries[start:end].to(keys.dtype), keys.transpose(0, 1))
-        probabilities, projection = _C.temporal_probabilities(
-            logits.contiguous(), projected, query_positions[start:end], key_positions,
-            1.0 / math.sqrt(keys.shape[-1]))
-        scores = _C.temporal_risk(probabilities, projection, projected, margin, candidate_start,
-                                  candidate_end, denominator_epsilon)
-        result = scores if result is None else torch.maximum(result, scores)
-    return result
+    return (_temporal_module or _temporal()).temporal_head_scores(
+        queries, query_positions, keys, key_positions, values, int(candidate_start),
+        int(candidate_end), margin_gradient, base_margin, float(denominator_epsilon), int(chunk))
+
+
+_temporal_module = None
+
+
+def _temporal():
+    """The C++ host module with the temporal operators bound (once): a head's chunk loop, its
+    library products and its launches run there."""
+    global _temporal_module
+    if _temporal_module is None:
+        import ctypes
+        planner, library = _planner(), _lib.load()
+        address = lambda name: ctypes.cast(getattr(library, name), ctypes.c_void_p).value
+        planner.bind_temporal(address("lr_temporal_probabilities"), address("lr_temporal_risk"),
+                              address("lr_temporal_risk_max"), address("lr_last_error"))
+        _temporal_module = planner
+    return _temporal_module
 
 
 def _planner():

@@ -60,6 +60,12 @@ int lr_temporal_risk(const float* probabilities, const float* output_projection,
                      const float* projected, const float* margin, int64_t window, int64_t groups,
                      int64_t length, int64_t first, int64_t last, double epsilon, float* result,
                      void* stream);
+/* The same, with result[i] = max(result[i], risk) (a NaN of either stays): a further chunk of a
+ * head's queries folded into the scores (torch.maximum over the chunks, scoring.py:192-194). */
+int lr_temporal_risk_max(const float* probabilities, const float* output_projection,
+                         const float* projected, const float* margin, int64_t window,
+                         int64_t groups, int64_t length, int64_t first, int64_t last,
+                         double epsilon, float* result, void* stream);
 
 /* append (csrc/scoring.cu:130-162, 264-292). keys/values [rows, dim], positions [rows] f32,
  * new_keys/new_values [1, heads, added, dim], cumulative [heads + 1] i32.

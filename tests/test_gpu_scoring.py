@@ -93,6 +93,44 @@ def test_temporal_ops_across_row_and_window_sizes(device, window, groups, length
     assert torch.isnan(blind).all()  # exp(-inf - -inf), as the definition has it
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("chunk", [1, 7, 64, 1000])
+def test_temporal_head_scores_equals_the_operators(device, dtype, chunk):
+    """The whole head in one native call gives the scores of the operators chunk by chunk, bit for
+    bit, in the forms the arguments may take: transposed queries, strided values, positions of
+    other shapes and types, a margin on the host, and a NaN in one key's value."""
+    window, groups, length, dim, first, last = 23, 3, 301, 64, 5, 290
+    queries = rand((groups, window, dim), dtype, device, 21).transpose(0, 1)
+    keys = rand((length, dim), dtype, device, 22)
+    values = rand((dim, length), dtype, device, 23).transpose(0, 1)
+    values[40, 3] = float("nan")
+    gradient = rand((groups, dim), torch.float32, device, 24).abs()
+    positions = torch.arange(length, device=device)
+    query_positions = torch.arange(length - window, length, device=device, dtype=torch.int32)
+
+    def by_operators():
+        projected = torch.matmul(gradient, values.float().transpose(0, 1)).contiguous()
+        result = None
+        for start in range(0, window, chunk):
+            logits = torch.matmul(queries[start:start + chunk], keys.transpose(0, 1))
+            p, out = _C.temporal_probabilities(logits.contiguous(), projected,
+                                               query_positions[start:start + chunk].long(),
+                                               positions.float(), 1.0 / math.sqrt(dim))
+            scores = _C.temporal_risk(p, out, projected, torch.tensor([2.0], device=device),
+                                      first, last, 1e-6)
+            result = scores if result is None else torch.maximum(result, scores)
+        return result
+
+    for value, finite in ((float("nan"), False), (0.5, True)):  # one NaN reaches every row
+        values[40, 3] = value
+        got = scoring.temporal_head_scores(queries, query_positions, keys, positions[:, None],
+                                           values, first, last, gradient, torch.tensor(2.0), 1e-6,
+                                           chunk)
+        expect = by_operators()
+        assert got.shape == (last - first,) and torch.isfinite(expect).all() == finite
+        torch.testing.assert_close(got, expect, rtol=0, atol=0, equal_nan=True)
+
+
 def test_temporal_risk_nonfinite(device):
     p = torch.full((3, 2, 10), 0.1, device=device)
     op = torch.zeros((3, 2), device=device)
