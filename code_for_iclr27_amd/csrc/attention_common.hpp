@@ -77,13 +77,39 @@ __device__ __forceinline__ attn_u32x4 load16(const void* p) {
   return *(const __attribute__((address_space(1))) attn_u32x4*)p;
 }
 
+// Index arithmetic is unsigned 32-bit (a call has fewer than 2^31 query rows and blocks): the 64-bit
+// divisions of a tile's coordinates took over a thousand instructions ahead of the first load.
+
+// Query of row `row` (row = query * G + group).
+__device__ __forceinline__ unsigned query_of(const AttnArgs& a, unsigned row) {
+  return a.length == 1 ? 0u : row / static_cast<unsigned>(a.groups);
+}
+
 // Output row `row` of segment `seg` (query i = row / G, query head h*G + row % G).
 template <typename T, int D>
-__device__ __forceinline__ T* output_row(const AttnArgs& a, int64_t seg, int64_t row) {
-  const int64_t b = seg / a.kv_heads, h = seg - b * a.kv_heads;
-  const int64_t i = row / a.groups, g = row - i * a.groups;
-  const int64_t heads = a.kv_heads * a.groups;
-  return static_cast<T*>(a.out) + ((b * a.length + i) * heads + h * a.groups + g) * D;
+__device__ __forceinline__ T* output_row(const AttnArgs& a, unsigned seg, unsigned row) {
+  const unsigned groups = static_cast<unsigned>(a.groups), kv_heads = static_cast<unsigned>(a.kv_heads);
+  const unsigned b = seg / kv_heads, h = seg - b * kv_heads;
+  const unsigned i = query_of(a, row), g = row - i * groups;
+  return static_cast<T*>(a.out) +
+         ((static_cast<int64_t>(b) * a.length + i) * (a.kv_heads * a.groups) + h * groups + g) * D;
+}
+
+// A value and its copy in the lane 16 (32) away, in both lanes: the row swap of two registers that
+// hold it, no LDS round trip. (Inline assembly: this compiler's builtin returns its first result
+// twice. The wait states cover a vector instruction that has just written the operands.)
+struct LanePair {
+  float first, second;
+};
+template <int DISTANCE>
+__device__ __forceinline__ LanePair lane_pair(float x) {
+  static_assert(DISTANCE == 16 || DISTANCE == 32, "row swaps");
+  float a = x, b = x;
+  if constexpr (DISTANCE == 16)
+    asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  else
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return {a, b};
 }
 
 // A (max, exp-sum, unnormalised output slice) softmax state; merge_into folds another in.

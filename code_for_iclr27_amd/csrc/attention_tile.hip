@@ -103,11 +103,10 @@ __device__ __forceinline__ tile_u32x2 read_transposed(uint32_t p) {
       (__attribute__((address_space(3))) tile_s16x4*)(uintptr_t)p));
 }
 
-// The larger of a value's copies in lanes l and l + 32, in both lanes (no LDS round trip).
+// The larger of a value's copies in lanes l and l + 32, in both lanes.
 __device__ __forceinline__ float both_halves_max(float x) {
-  const unsigned bits = __builtin_bit_cast(unsigned, x);
-  const auto swapped = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-  return fmaxf(__builtin_bit_cast(float, swapped[0]), __builtin_bit_cast(float, swapped[1]));
+  const LanePair pair = lane_pair<32>(x);
+  return fmaxf(pair.first, pair.second);
 }
 
 // The tile's place in its segment: bounds clamped into the key buffer as in attention.hip.

@@ -150,11 +150,11 @@ def test_prefill_masked_keys_never_contribute(device, dim, groups, history):
     assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
 
 
-@pytest.mark.parametrize("scale", [0.0, -0.125, 0.5])
+@pytest.mark.parametrize("scale", [0.0, -0.125, 0.5, 2.0])
 def test_prefill_scales_through_the_abi(device, scale):
     """lr_packed_attention's scale is any number: zero (the mean of the visible values) and
-    negative ones too. A larger scale has a larger relative rounding of the f32 exponent, so
-    0.5 at d64 (logits up to 20) still fits the same tolerance."""
+    negative ones too. A larger scale has a larger relative rounding of the f32 exponents:
+    2^-24 of logits up to 90 (scale 2 at d64) is 6e-6 of a probability, within the tolerance."""
     from code_for_iclr27_amd import _lib
     length, kv_heads, groups, dim = 50, 2, 4, 64
     q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim, [50, 120], seed=19)
