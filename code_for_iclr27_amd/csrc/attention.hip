@@ -41,11 +41,62 @@ constexpr int kSmallWaveKeys = 16;
 constexpr int64_t kFewBlocks = 512;
 // Partial states the allocation-free entry point holds (per device).
 constexpr size_t kAttentionScratchBytes = size_t{16} << 20;
-// Partial blocks each merging thread loads at once: four, or twelve where a thread folds more
-// than four blocks (batch-1 decode: cfg1's 36 blocks per unit take one round of loads instead
-// of three; measured 14.9 against 15.3 us per layer, and no better for cfg2's 12 blocks).
-constexpr int kMergeUnroll = 4;
-constexpr int kMergeUnrollWide = 12;
+
+// The value of the lane a reduction step pairs with. Lane bits 0 and 1: that lane exactly; bits 2
+// and 3: a lane of the other half of 8 or 16 lanes, the same value once the bits below are
+// reduced (cross-lane reads in the vector ALU, no LDS round trip).
+template <int BIT>
+__device__ __forceinline__ float paired(float x) {
+  constexpr int kControl = BIT == 0 ? 0xB1 : BIT == 1 ? 0x4E : BIT == 2 ? 0x141 : 0x140;
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+      0, __builtin_bit_cast(int, x), kControl, 0xF, 0xF, false));
+}
+// Max or sum over the 16 lanes of a row, in all of them.
+template <bool kMax>
+__device__ __forceinline__ float reduce16(float x) {
+  auto step = [&](float y) { x = kMax ? fmaxf(x, y) : x + y; };
+  step(paired<0>(x));
+  step(paired<1>(x));
+  step(paired<2>(x));
+  step(paired<3>(x));
+  return x;
+}
+// x plus its copy in the lane 2^BIT away (BIT 3: see paired; 4 and 5 swap whole rows).
+template <int BIT>
+__device__ __forceinline__ float plus_paired(float x) {
+  if constexpr (BIT <= 3) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                   0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false));  // row_ror:8
+  } else {
+    const LanePair pair = lane_pair<1 << BIT>(x);
+    return pair.first + pair.second;
+  }
+}
+
+// Segment bounds, clamped into the key buffer, and the key blocks (of `block` keys) that the tile
+// whose last query is `last_query` sees. A pending row (the decode step's own token, not yet
+// appended) is key `cached` of the segment, after its cached rows.
+struct SegmentKeys {
+  int64_t key0;
+  int cached, n, shift, key_end, needed;  // query i sees keys j <= i + shift
+};
+__device__ __forceinline__ SegmentKeys segment_keys(const AttnArgs& a, unsigned seg,
+                                                    unsigned last_query, int block) {
+  SegmentKeys k;
+  int64_t key0 = a.cu[seg], n = static_cast<int64_t>(a.cu[seg + 1]) - key0;
+  key0 = key0 < 0 ? 0 : (key0 > a.key_rows ? a.key_rows : key0);
+  n = n < 0 ? 0 : (n > a.key_rows - key0 ? a.key_rows - key0 : n);
+  k.key0 = key0;
+  k.cached = static_cast<int>(n);
+  k.n = k.cached + (a.pending_keys != nullptr ? 1 : 0);
+  k.shift = k.n - static_cast<int>(a.length);
+  const int end = static_cast<int>(last_query) + k.shift + 1;
+  k.key_end = end < 0 ? 0 : (end > k.n ? k.n : end);
+  // keys past splits * block are not read
+  k.needed = min(static_cast<int>((static_cast<unsigned>(k.key_end) + block - 1) / block),
+                 static_cast<int>(a.splits));
+  return k;
+}
 
 template <typename T, int D, int R, int CH>
 __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attention_kernel(AttnArgs a) {
@@ -66,28 +117,17 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
   __shared__ float wave_ml[kAttnWaves][R][2];
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int64_t unit = blockIdx.x / a.splits, split = blockIdx.x - unit * a.splits;
-  const int64_t seg = unit / a.tiles, tile = unit - seg * a.tiles;
-  const int64_t rows = a.length * a.groups;
-  const int64_t row0 = tile * R;
-  const int64_t rows_here = rows - row0 < R ? rows - row0 : R;
+  const unsigned splits = static_cast<unsigned>(a.splits), tiles = static_cast<unsigned>(a.tiles);
+  const unsigned groups = static_cast<unsigned>(a.groups);
+  const unsigned unit = blockIdx.x / splits, split = blockIdx.x - unit * splits;
+  const unsigned seg = tiles == 1 ? unit : unit / tiles, tile = unit - seg * tiles;
+  const unsigned rows = static_cast<unsigned>(a.length) * groups;
+  const unsigned row0 = tile * R;
+  const int rows_here = static_cast<int>(min(rows - row0, static_cast<unsigned>(R)));
+  constexpr int kBlockKeys = kAttnWaves * CH;
+  const SegmentKeys keys = segment_keys(a, seg, query_of(a, row0 + rows_here - 1), kBlockKeys);
 
-  // Segment bounds, clamped into the key buffer. A pending row (the decode step's own token,
-  // not yet appended) is key `cached` of the segment, after its cached rows.
-  int64_t key0 = a.cu[seg], n = static_cast<int64_t>(a.cu[seg + 1]) - key0;
-  key0 = key0 < 0 ? 0 : (key0 > a.key_rows ? a.key_rows : key0);
-  n = n < 0 ? 0 : (n > a.key_rows - key0 ? a.key_rows - key0 : n);
-  const int64_t cached = n;
-  if (a.pending_keys != nullptr) ++n;
-  const int64_t shift = n - a.length;  // query i sees keys j <= i + shift
-  const int64_t last_query = (row0 + rows_here - 1) / a.groups;
-  int64_t key_end = last_query + shift + 1;
-  key_end = key_end < 0 ? 0 : (key_end > n ? n : key_end);
-  constexpr int64_t kBlockKeys = kAttnWaves * CH;
-  int64_t needed = (key_end + kBlockKeys - 1) / kBlockKeys;
-  needed = needed > a.splits ? a.splits : needed;  // keys past splits * block keys are not read
-
-  if (needed == 0) {  // no visible key for any row of this tile: zeros
+  if (keys.needed == 0) {  // no visible key for any row of this tile: zeros
     if (split != 0) return;
     for (int item = tid; item < ITEMS; item += kAttnThreads) {
       const int r = item / LPK, c = item - r * LPK;
@@ -97,11 +137,11 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     }
     return;
   }
-  if (split >= needed) return;  // uniform across the workgroup
+  if (static_cast<int>(split) >= keys.needed) return;  // uniform across the workgroup
 
-  const int64_t kb = split * kBlockKeys + wave * CH;
-  const int64_t ke = kb + CH < key_end ? kb + CH : key_end;
-  const int nk = kb < ke ? static_cast<int>(ke - kb) : 0;
+  const int kb = static_cast<int>(split) * kBlockKeys + wave * CH;
+  const int ke = kb + CH < keys.key_end ? kb + CH : keys.key_end;
+  const int nk = kb < ke ? ke - kb : 0;
   const int m = lane & 15, j = lane >> 4;
   const int kg = lane / LPK, c = lane - kg * LPK;
 
@@ -114,24 +154,25 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
 
   if (nk > 0) {
-    const T* kbase = static_cast<const T*>(a.keys) + (key0 + kb) * D;
-    const T* vbase = static_cast<const T*>(a.values) + (key0 + kb) * D;
+    const T* kbase = static_cast<const T*>(a.keys) + (keys.key0 + kb) * D;
+    const T* vbase = static_cast<const T*>(a.values) + (keys.key0 + kb) * D;
     // row of wave key `key` (< nk): a cached row, or the segment's pending row
-    const int64_t cached_here = cached - kb;
+    const int cached_here = keys.cached - kb;
     auto key_row = [&](const T* base, const void* pending, int key) -> const T* {
-      return key < cached_here ? base + static_cast<int64_t>(key) * D
-                               : static_cast<const T*>(pending) + seg * D;
+      return key < cached_here ? base + key * D
+                               : static_cast<const T*>(pending) + static_cast<int64_t>(seg) * D;
     };
     // Every load of the wave is issued before the first use: queries (A operand, row m = lane
     // & 15, k chunk j = lane >> 4), K rows (B operand, key m of each 16-key block), V slices.
     X8 qop[KS];
     {
       const bool row_ok = m < rows_here;
-      const int64_t row = row0 + (row_ok ? m : 0);
-      const int64_t b = seg / a.kv_heads, h = seg - b * a.kv_heads;
-      const int64_t i = row / a.groups, g = row - i * a.groups;
+      const unsigned row = row0 + (row_ok ? m : 0);
+      const unsigned b = seg / static_cast<unsigned>(a.kv_heads);
+      const unsigned h = seg - b * static_cast<unsigned>(a.kv_heads);
+      const unsigned i = query_of(a, row), g = row - i * groups;
       const T* q = static_cast<const T*>(a.queries) + b * a.q_batch +
-                   (h * a.groups + g) * a.q_head + i * a.q_query + 8 * j;
+                   static_cast<int64_t>(h * groups + g) * a.q_head + i * a.q_query + 8 * j;
       // Unconditional loads from a valid row (padding lanes read row0's) and a select after
       // them: a load under a branch is waited for inside the branch.
       attn_u32x4 raw[KS];
@@ -159,12 +200,11 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     }
 
     // QK^T. D layout: lane holds key 16 * blk + (lane & 15) for rows 4j + r.
-    int64_t limit[4];  // causal limit of this lane's rows, relative to kb (keys <= limit seen)
+    int limit[4];  // causal limit of this lane's rows, relative to kb (keys <= limit seen)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = row0 + 4 * j + r;
-      limit[r] = (4 * j + r < rows_here) ? row / a.groups + shift - kb : -1;
-    }
+    for (int r = 0; r < 4; ++r)
+      limit[r] = 4 * j + r < rows_here
+                     ? static_cast<int>(query_of(a, row0 + 4 * j + r)) + keys.shift - kb : -1;
     float s[NB][4];
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk) {
@@ -180,10 +220,7 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     }
     // Row max and exp-sum over the 16 lanes that share rows 4j .. 4j + 3.
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int offset = 1; offset < 16; offset <<= 1)
-        row_max[r] = fmaxf(row_max[r], __shfl_xor(row_max[r], offset));
+    for (int r = 0; r < 4; ++r) row_max[r] = reduce16<true>(row_max[r]);
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk) {
       attn_f32x4 p;
@@ -196,9 +233,7 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
       if (4 * j < R) *reinterpret_cast<attn_f32x4*>(&probs[wave][blk * 16 + m][4 * j]) = p;
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int offset = 1; offset < 16; offset <<= 1) row_sum[r] += __shfl_xor(row_sum[r], offset);
+    for (int r = 0; r < 4; ++r) row_sum[r] = reduce16<false>(row_sum[r]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -219,11 +254,13 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     }
     // Sum the KPI lane groups (lanes c, c + LPK, ... hold the same elements).
 #pragma unroll
-    for (int offset = LPK; offset < 64; offset <<= 1)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[r][e] += __shfl_xor(acc[r][e], offset);
+      for (int e = 0; e < 8; ++e) {
+        if constexpr (LPK <= 8) acc[r][e] = plus_paired<3>(acc[r][e]);
+        if constexpr (LPK <= 16) acc[r][e] = plus_paired<4>(acc[r][e]);
+        acc[r][e] = plus_paired<5>(acc[r][e]);
+      }
   }
 
   // Wave states to LDS: rows r = 4j + i are held by lanes 16j .. 16j + 15.
@@ -256,7 +293,7 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
       merge_into(st, wave_ml[w][r_item][0], wave_ml[w][r_item][1], o);
     }
   }
-  if (needed == 1) {  // the only block of keys: normalise and write
+  if (keys.needed == 1) {  // the only block of keys: normalise and write
     if (tid < ITEMS && r_item < rows_here) {
       const float inv = st.l > 0.f ? 1.0f / st.l : 0.f;
       float o[8];
@@ -269,7 +306,7 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
   }
 
   // ---- Partial state of this block; attention_merge_kernel combines the blocks.
-  const int64_t slot = (unit * a.splits + split) * R;
+  const int64_t slot = static_cast<int64_t>(blockIdx.x) * R;
   if (tid < ITEMS) {
     float* po = a.part_o + (slot + r_item) * D + 8 * c_item;
     *reinterpret_cast<attn_f32x4*>(po) = attn_f32x4{st.o[0], st.o[1], st.o[2], st.o[3]};
@@ -290,49 +327,46 @@ __global__ __launch_bounds__(kAttnThreads) void attention_merge_kernel(AttnArgs 
   constexpr int LPK = D / 8;
   constexpr int ITEMS = R * LPK;
   constexpr int PARTS = kAttnThreads / ITEMS;
-  constexpr int64_t kBlockKeys = kAttnWaves * CH;
   __shared__ __align__(16) float merge_o[kAttnThreads][8];
   __shared__ float merge_ml[kAttnThreads][2];
   const int tid = threadIdx.x;
-  const int64_t unit = blockIdx.x;
-  const int64_t seg = unit / a.tiles, tile = unit - seg * a.tiles;
-  const int64_t rows = a.length * a.groups;
-  const int64_t row0 = tile * R;
-  const int64_t rows_here = rows - row0 < R ? rows - row0 : R;
-  int64_t key0 = a.cu[seg], n = static_cast<int64_t>(a.cu[seg + 1]) - key0;
-  key0 = key0 < 0 ? 0 : (key0 > a.key_rows ? a.key_rows : key0);
-  n = n < 0 ? 0 : (n > a.key_rows - key0 ? a.key_rows - key0 : n);
-  if (a.pending_keys != nullptr) ++n;  // the pending row, as in the first launch
-  const int64_t last_query = (row0 + rows_here - 1) / a.groups;
-  int64_t key_end = last_query + n - a.length + 1;
-  key_end = key_end < 0 ? 0 : (key_end > n ? n : key_end);
-  int64_t needed = (key_end + kBlockKeys - 1) / kBlockKeys;
-  needed = needed > a.splits ? a.splits : needed;
-  if (needed <= 1) return;  // the first launch wrote this tile's output
-
+  const unsigned unit = blockIdx.x, tiles = static_cast<unsigned>(a.tiles);
+  const unsigned splits = static_cast<unsigned>(a.splits);
+  const unsigned seg = tiles == 1 ? unit : unit / tiles, tile = unit - seg * tiles;
+  const unsigned rows = static_cast<unsigned>(a.length) * static_cast<unsigned>(a.groups);
+  const unsigned row0 = tile * R;
+  const int rows_here = static_cast<int>(min(rows - row0, static_cast<unsigned>(R)));
   const int part = tid / ITEMS, item = tid - part * ITEMS;
   const int r = item / LPK, cc = item - r * LPK;
-  const int64_t first = unit * a.splits * R;
-  MergeState total{kNegInf, 0.f, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
-  for (int64_t k0 = part; k0 < needed; k0 += PARTS * U) {
-    float mk[U], lk[U];
-    attn_f32x4 lo[U], hi[U];
+  const int64_t first = static_cast<int64_t>(unit) * splits * R;
+  // The first round of partial states is loaded before the segment's bounds are known (every slot
+  // of the grid's splits is in the workspace; those past the needed ones are not used), so that
+  // the two memory round trips overlap.
+  float mk[U], lk[U];
+  attn_f32x4 lo[U], hi[U];
+  auto load = [&](unsigned k0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      int64_t k = k0 + u * PARTS;
-      const bool live = k < needed;
-      k = live ? k : k0;
-      const int64_t at = first + k * R + r;
-      mk[u] = live ? a.part_ml[at * 2] : kNegInf;
+      const unsigned k = k0 + u * PARTS < splits ? k0 + u * PARTS : 0;
+      const int64_t at = first + static_cast<int64_t>(k) * R + r;
+      mk[u] = a.part_ml[at * 2];
       lk[u] = a.part_ml[at * 2 + 1];
       lo[u] = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * cc);
       hi[u] = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * cc + 4);
     }
+  };
+  load(part);
+  const unsigned needed = static_cast<unsigned>(
+      segment_keys(a, seg, query_of(a, row0 + rows_here - 1), kAttnWaves * CH).needed);
+  if (needed <= 1) return;  // the first launch wrote this tile's output
+  MergeState total{kNegInf, 0.f, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+  for (unsigned k0 = part; k0 < needed; k0 += PARTS * U) {
+    if (k0 != static_cast<unsigned>(part)) load(k0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float o[8] = {lo[u][0], lo[u][1], lo[u][2], lo[u][3],
                           hi[u][0], hi[u][1], hi[u][2], hi[u][3]};
-      merge_into(total, mk[u], lk[u], o);
+      merge_into(total, k0 + u * PARTS < needed ? mk[u] : kNegInf, lk[u], o);
     }
   }
 #pragma unroll
@@ -391,7 +425,7 @@ size_t workspace_bytes(const AttnPlan& p, int64_t dim) {
 // keys, 8 queries: 35.1 against 23.1 us). At d64 the tiles are already ahead (2 queries on 500
 // keys 9.1 against 11.5 us, 8 on 4000 14.9 against 32.8).
 bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys, int64_t dim) {
-  if (length <= 1 || length > INT32_MAX / groups) return false;
+  if (length <= 1) return false;
   const bool few_rows = length * groups <= 32;
   return dim == 64 || !few_rows || max_keys <= 128 || max_keys > 40000 / segments;
 }
@@ -412,16 +446,20 @@ int launch_attention(const AttnArgs& args, int64_t blocks, hipStream_t stream) {
                      dim3(kAttnThreads), 0, stream, args);
   if (int status = check_launch("packed_attention")) return status;
   if (args.splits == 1) return LR_OK;
-  // blocks each merging thread folds: PARTS = threads / (R * D / 8) threads share a row slice
+  // Blocks each merging thread folds (PARTS = threads / (R * D / 8) threads share a row slice):
+  // the smallest round of loads that holds them, or rounds of twelve. Nine of a cfg1 layer's 36
+  // blocks in a round of nine take 0.6 us a layer less than in one of twelve, whose last loads
+  // repeat a block.
   const int64_t per_part = ceil_div(args.splits, int64_t{kAttnThreads / (R * D / 8)});
-  if (per_part > kMergeUnroll)
-    hipLaunchKernelGGL((attention_merge_kernel<T, D, R, CH, kMergeUnrollWide>),
-                       dim3(static_cast<unsigned>(blocks / args.splits)), dim3(kAttnThreads), 0,
-                       stream, args);
-  else
-    hipLaunchKernelGGL((attention_merge_kernel<T, D, R, CH, kMergeUnroll>),
-                       dim3(static_cast<unsigned>(blocks / args.splits)), dim3(kAttnThreads), 0,
-                       stream, args);
+  auto merge = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks / args.splits)),
+                       dim3(kAttnThreads), 0, stream, args);
+  };
+  if (per_part <= 2) merge(attention_merge_kernel<T, D, R, CH, 2>);
+  else if (per_part <= 4) merge(attention_merge_kernel<T, D, R, CH, 4>);
+  else if (per_part <= 6) merge(attention_merge_kernel<T, D, R, CH, 6>);
+  else if (per_part <= 9) merge(attention_merge_kernel<T, D, R, CH, 9>);
+  else merge(attention_merge_kernel<T, D, R, CH, 12>);
   return check_launch("packed_attention merge");
 }
 
@@ -479,6 +517,7 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
   LR_REQUIRE(pending_keys == nullptr || length == 1, "Pending rows need one query per segment");
   LR_REQUIRE(dim == 64 || dim == 128 || dim == 256, "Head dimension must be 64, 128 or 256");
   LR_REQUIRE(batch > 0 && kv_heads > 0 && groups > 0 && length > 0, "Empty attention dimensions");
+  LR_REQUIRE(length <= INT32_MAX / groups, "Attention grid too large");
   LR_REQUIRE(key_rows >= 0 && max_keys >= 0, "Invalid key lengths");
   LR_REQUIRE(queries && out && cu_seqlens_k && (key_rows == 0 || (keys && values)),
              "Invalid attention buffers");
