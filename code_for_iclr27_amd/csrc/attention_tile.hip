@@ -204,14 +204,18 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
   const __bf16* keys = static_cast<const __bf16*>(a.keys) + bounds.key0 * D;
   const __bf16* values = static_cast<const __bf16*>(a.values) + bounds.key0 * D;
   const uint32_t k_base = lds_address(&k_lds[0][0]), v_base = lds_address(&v_lds[0][0]);
-  const uint32_t k_offset = dma_row_offset<D, RowSwizzle<D>, kThreads>();
+  // d256 keeps 8 chunk slots: with 16 the copies' offsets differ from row group to row group, and
+  // the bank conflicts they would save are hidden here (1000 queries onto 4000 cached keys, 4 heads
+  // x 6 groups: 234.5 us with 8, 237.7 with 16).
+  using KeySwizzle = RowSwizzle<D, D == 128 ? 16 : 8>;
+  const uint32_t k_offset = dma_row_offset<D, KeySwizzle, kThreads>();
   const uint32_t v_offset = dma_row_offset<D, ColumnSwizzle<D>, kThreads>();
   constexpr uint32_t kStageBytes = KEYS * D * 2;
   // Rows past the last visible key re-read it (masked). K runs one stage ahead of V; `at` is the
   // byte offset of the stage's buffer.
   auto fetch_k = [&](int key, uint32_t at) {
-    dma_rows<D, KEYS, RowSwizzle<D>, kThreads>(keys, key, bounds.key_end - 1,
-                                               k_base + at, k_offset);
+    dma_rows<D, KEYS, KeySwizzle, kThreads>(keys, key, bounds.key_end - 1,
+                                            k_base + at, k_offset);
   };
   auto fetch_v = [&](int key, uint32_t at) {
     dma_rows<D, KEYS, ColumnSwizzle<D>, kThreads>(values, key, bounds.key_end - 1,
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       acc = Vec::mfma(*reinterpret_cast<const attn_u32x4*>(
-                          k_row + 16 * swizzled_chunk<D>(col, half * KS + ks)),
+                          k_row + 16 * KeySwizzle::slot(col, half * KS + ks)),
                       qop[ks], acc);
     return acc;
   };
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
       float p[16], part = 0.0f;
       auto load_k = [&](int ks) {
         k_op[ks] = *reinterpret_cast<const attn_u32x4*>(
-            k_row + 16 * swizzled_chunk<D>(col, half * KS + ks));
+            k_row + 16 * KeySwizzle::slot(col, half * KS + ks));
       };
       auto load_v = [&](int k, int dt) {  // 16 keys: accumulators 8k .. 8k + 7
         const uint32_t at = v_lane[dt] + here + 16 * k * (D * 2);

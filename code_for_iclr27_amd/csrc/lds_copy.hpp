@@ -1,5 +1,6 @@
 // Direct global -> LDS copies and swizzled LDS tiles of 16-bit rows, shared by the kernels that
-// stage K, V or Q tiles (scorer.hip, attention_tile.hip). Workgroups of 256 threads.
+// stage K, V, Q or weight tiles (scorer.hip, attention_tile.hip, vjp_products.hip), by whole
+// workgroups or by single waves.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -78,25 +79,27 @@ __device__ __forceinline__ void dma_wait_but() {
   asm volatile("" ::: "memory");
 }
 
-// Swizzled LDS rows: D bf16 per row, no padding; 16-byte chunk c of row r is stored in chunk
-// slot c ^ (r % P), so the lanes that read chunk c of consecutive rows (an MFMA operand) touch
-// P different 16-byte bank groups per P rows. P = 16 for d = 128 (its 16 chunks per row allow
-// it; measured 2% faster in the row pass than P = 8), else 8.
+// Swizzled LDS rows: D 16-bit elements per row, no padding; 16-byte chunk c of row r is stored in
+// chunk slot c ^ (r % P), so the lanes that read chunk c of consecutive rows (an MFMA operand)
+// touch P different 16-byte bank groups per P rows. P = 16 where a row has the chunks for it
+// (d64 has 8): then 16 rows' chunks touch all 64 banks once. With P = 8 at d256 four of every
+// twelve LDS cycles of the audit were conflicts, with 16 there are none (row pass over 9216 keys,
+// 16 layers x 4 heads x 6 groups, window 512: 945 -> 914 us).
 template <int D>
-constexpr int swizzle_period() { return D == 128 ? 16 : 8; }
+constexpr int swizzle_period() { return D == 64 ? 8 : 16; }
 
-template <int D>
+template <int D, int P = swizzle_period<D>()>
 __device__ __forceinline__ int swizzled_chunk(int row, int chunk) {
-  return chunk ^ (row & (swizzle_period<D>() - 1));
+  return chunk ^ (row & (P - 1));
 }
 
 // The swizzles a copy can apply: rows read as MFMA operand rows (above), or read transposed
 // (ds_read_b64_tr_b16: 16 lanes take 4 consecutive rows x 16 columns, 4 x 32 bytes). For the
 // latter, 64-byte blocks of four consecutive rows go to the four 64-byte quarters of the 64
 // banks, so that 32 lanes' reads (4 rows x 64 bytes) touch every bank once.
-template <int D>
+template <int D, int P = swizzle_period<D>()>
 struct RowSwizzle {
-  static __device__ __forceinline__ int slot(int row, int chunk) { return swizzled_chunk<D>(row, chunk); }
+  static __device__ __forceinline__ int slot(int row, int chunk) { return swizzled_chunk<D, P>(row, chunk); }
 };
 template <int D>
 struct ColumnSwizzle {
@@ -106,11 +109,14 @@ struct ColumnSwizzle {
 };
 
 // DMA of `ROWS` consecutive rows (row0..) of a 16-bit matrix, D elements of each (`stride` elements
-// from row to row: D, or a multiple of 128), into swizzled LDS rows at LDS byte address `lds`; rows at or past `last_row` re-read row `last_row` (callers mask them; no CLAMP: there are none). All
-// THREADS threads of the workgroup call it, or, with 64, one wave (with its lane as `thread`). Copy i moves rows [i * RPI, (i + 1) * RPI), RPI =
-// THREADS / (D / 8): while every row lies before `last_row` the addresses are a scalar base plus
-// the thread's byte offset within copy 0 (`dma_row_offset`), its chunk exchanged with what the
-// swizzle does to row i * RPI (nothing where RPI is a multiple of the swizzle's period).
+// from row to row: D, or a multiple of 128), into swizzled LDS rows at LDS byte address `lds`; rows
+// at or past `last_row` re-read row `last_row` (callers mask them; no CLAMP: there are none). All
+// THREADS threads of the workgroup call it, or, with 64, one wave (with its lane as `thread`).
+// Copy i moves rows [i * RPI, (i + 1) * RPI), RPI = THREADS / (D / 8): while every row lies before
+// `last_row` the addresses are a scalar base plus the thread's byte offset within copy 0
+// (`dma_row_offset`), its chunk exchanged with what the swizzle does to row i * RPI (nothing where
+// RPI is a multiple of the swizzle's period; the swizzle is an exclusive or of row bits, so the
+// two parts of the row combine).
 template <int D, typename Swizzle = RowSwizzle<D>, int THREADS = 256>
 __device__ __forceinline__ uint32_t dma_row_offset(int thread = threadIdx.x, int stride = D) {
   constexpr int CH = D / 8;
