@@ -12,8 +12,12 @@
 //
 // Precision. P is f32 and stays f32: it enters the 16-bit MFMA as a sum of 16-bit pieces whose
 // products with V are exact in f32. bf16: three pieces by truncation, 3 x 8 bits = the whole
-// 24-bit significand. f16: two pieces by rounding, 11 + 11 bits and the residual's sign, f32's own
-// half-ulp, with P scaled by 2^7 so that the pieces of small P stay clear of f16's subnormals.
+// 24-bit significand. f16: pieces by rounding. With P scaled by 2^11 two of them hold 11 + 11 bits
+// and a sign, but nothing below 2^-25 (f16's subnormals), which is 2^-12 of P = 2^-24. So what they
+// leave goes, 2^24 times larger, into two more pieces (the tails) whose products are summed apart
+// and added to the output once a stage. The four are within 2^-60 of P (all of its bits down to
+// 2^-36 of the reference): n keys are within 2^-44 n of the sum with f32 P, for any f16 V, against
+// output steps of 2^-24 and more.
 //
 // The reference of a row's exponentials only moves when the row's maximum has outgrown it by
 // 2^kSlack (the accumulators are rescaled then, seldom after the first stages); sums and products
@@ -23,9 +27,11 @@
 // and wave at d128, with about 170 vector instructions beside them. Measured (us, against the
 // split-key kernel of attention.hip, whose 8-row tiles read every K and V row once each and
 // multiply P*V on the VALU): 8192 queries of the 8B shape 883 against 10,878 (1.25 PFLOP/s of
-// MFMA work), 1000 queries on 4,000 cached keys at d256, G6, 233 against 2,115; 333 queries at
-// d64, f16, 10.6 against 24.3. Three waves per SIMD (168 VGPRs, a few spills outside the loop)
-// beat two without spills at d <= 128: 890 against 928. d256 holds one wave per SIMD (its
+// MFMA work), 1000 queries on 4,000 cached keys at d256, G6, 233 against 2,115. f16: 333 queries
+// at d64 15.4 against 24.3, 8192 at d128 1,140 against 10,768 (two pieces without the tails, which
+// lose the small P, 10.6 and 772; V as two bf16 pieces, six products, 15.3 and 1,717). Three waves
+// per SIMD (168 VGPRs, a few spills outside the loop) beat two without spills at d <= 128: 890
+// against 928 (f16 at d128, with the tails' accumulators, holds two). d256 holds one wave per SIMD (its
 // accumulators alone take 128 VGPRs), so its stream is laid out by hand: 233 against 285.
 // Stages of 64 keys, a third stage buffer, 32-row tiles for long prompts: no faster or slower.
 //
@@ -56,7 +62,7 @@ constexpr int kBuffers = 2;     // K and V stages in LDS
 
 template <typename T> struct TileVec;
 template <> struct TileVec<__bf16> {
-  static constexpr int kPieces = 3;
+  static constexpr int kPieces = 3, kTails = 0;
   static constexpr float kRaise = 0.0f;
   static __device__ __forceinline__ tile_f32x16 mfma(attn_u32x4 a, attn_u32x4 b, tile_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(attn_bf16x8, a),
@@ -77,19 +83,26 @@ template <> struct TileVec<__bf16> {
   }
 };
 template <> struct TileVec<_Float16> {
-  static constexpr int kPieces = 2;
-  static constexpr float kRaise = 7.0f;  // P <= 2^(kSlack + 7), far from f16's 65504
+  static constexpr int kPieces = 2, kTails = 2;
+  static constexpr float kRaise = 11.0f;  // P <= 2^(kSlack + 11), half of f16's range
+  static constexpr float kTailScale = 0x1p24f;
   static __device__ __forceinline__ tile_f32x16 mfma(attn_u32x4 a, attn_u32x4 b, tile_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(attn_f16x8, a),
                                                   __builtin_bit_cast(attn_f16x8, b), c, 0, 0, 0);
   }
-  static __device__ __forceinline__ void split(float x, float y, attn_u32x4 (&piece)[2], int w) {
+  // Each piece rounds what the ones before have left (exact differences); the tails are pieces of
+  // 2^24 times the rest, which is at most 2^-24 of x or 2^-25.
+  static __device__ __forceinline__ void split(float x, float y, attn_u32x4 (&piece)[4], int w) {
     typedef _Float16 half2 __attribute__((ext_vector_type(2)));
-    const half2 high = {static_cast<_Float16>(x), static_cast<_Float16>(y)};
-    const half2 low = {static_cast<_Float16>(x - static_cast<float>(high[0])),
-                       static_cast<_Float16>(y - static_cast<float>(high[1]))};
-    piece[0][w] = __builtin_bit_cast(unsigned, high);
-    piece[1][w] = __builtin_bit_cast(unsigned, low);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i == kPieces) x *= kTailScale, y *= kTailScale;
+      const half2 part = {static_cast<_Float16>(x), static_cast<_Float16>(y)};
+      piece[i][w] = __builtin_bit_cast(unsigned, part);
+      if (i == 3) break;
+      x -= static_cast<float>(part[0]);
+      y -= static_cast<float>(part[1]);
+    }
   }
 };
 
@@ -133,7 +146,8 @@ __device__ __forceinline__ int chunks_needed(int key_end, int chunk, int splits)
 }
 
 template <typename T, int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D == 256 || WAVES == 1 ? 1 : 3))) void prefill_attention_kernel(
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
+    D == 256 || WAVES == 1 ? 1 : D == 128 && TileVec<T>::kTails > 0 ? 2 : 3))) void prefill_attention_kernel(
     AttnArgs a, unsigned segments, int chunk) {
   using Vec = TileVec<T>;
   constexpr int KEYS = kStageKeys;
@@ -309,7 +323,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
 #pragma unroll
       for (int r = 0; r < 16; ++r) next[r] = 0.0f;
       const char* k_row = reinterpret_cast<const char*>(&k_lds[0][0]) + ahead + col * (D * 2);
-      attn_u32x4 k_op[KS], v_op[2][DT], piece[2][Vec::kPieces];
+      attn_u32x4 k_op[KS], v_op[2][DT], piece[2][Vec::kPieces + Vec::kTails];
       float p[16], part = 0.0f;
       auto load_k = [&](int ks) {
         k_op[ks] = *reinterpret_cast<const attn_u32x4*>(
@@ -337,6 +351,24 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
       float top = kNegInf;
       auto product = [&](int k, int i) {
         out[i % DT] = Vec::mfma(v_op[k][i % DT], piece[k][i / DT], out[i % DT]);
+      };
+      // The tails' products with all 32 keys, by column tiles.
+      auto add_tails = [&]() {
+        if constexpr (Vec::kTails > 0) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            tile_f32x16 tail;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tail[r] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 2 * Vec::kTails; ++i)
+              tail = Vec::mfma(v_op[i / Vec::kTails][dt],
+                               piece[i / Vec::kTails][Vec::kPieces + i % Vec::kTails], tail);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              out[dt][r] = __builtin_fmaf(tail[r], 1.0f / Vec::kTailScale, out[dt][r]);
+          }
+        }
       };
       if constexpr (kLaidOut) {
         constexpr int kLead = KS < 4 ? KS : 4;
@@ -368,6 +400,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
             top = fmaxf(fmaxf(top, next[2 * r]), next[2 * r + 1]);
           __builtin_amdgcn_sched_barrier(0);
         }
+        add_tails();
       } else {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -383,6 +416,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(D ==
 #pragma unroll
           for (int i = 0; i < kProducts; ++i) product(k, i);
         }
+        add_tails();
 #pragma unroll
         for (int r = 0; r < 8; ++r) top = fmaxf(fmaxf(top, next[2 * r]), next[2 * r + 1]);
       }

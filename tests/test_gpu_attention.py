@@ -128,6 +128,33 @@ def test_prefill_tiles(device, dtype, batch, kv_heads, groups, length, dim, leng
     check(run(device, q, k, v, meta, length, kv_heads), q, k, v, cu, kv_heads)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups,length,dim,keys", [(4, 40, 64, 90), (4, 11, 128, 300),
+                                                    (6, 64, 256, 400), (1, 1, 64, 400)])
+def test_small_probabilities_keep_their_precision(device, dtype, groups, length, dim, keys):
+    """A dominant key with V = 0 and every other probability between 2^-27 and 2^-22 of it on
+    large values: the outputs are sums of small P times V alone, as accurate as any other. In f32
+    a small P carries its exponent's rounding (|exponent| < 32 here: 2^-20 ln 2, plus that of the
+    scale and of the reference), under 2^-16 of the sum of P |V|."""
+    q, k, v, cu, meta = make(device, 1, 2, groups, length, dim, [keys, keys], dtype, seed=23)
+    g = torch.Generator().manual_seed(24)
+    q *= 2.0 ** -4  # the other dimensions' share of a score stays small
+    q[..., 0] = 8.0
+    per_unit = 8.0 * dim ** -0.5 * np.log2(np.e)  # exponents of two for one unit of k[:, 0]
+    down = 22 + 5 * torch.rand(k.shape[0], generator=g)
+    k[:, 0] = (-down / per_unit).to(dtype)
+    v *= 2.0 ** 13
+    k[cu[:-1]], v[cu[:-1]] = 0.0, 0.0
+    arrays = [t.float().numpy() for t in (q, k, v)]
+    expect = oattention.packed_attention(*arrays, cu, 2)
+    total = oattention.packed_attention(*arrays[:2], np.abs(arrays[2]), cu, 2)
+    assert 1e-4 < np.abs(expect).max() < 1
+    got = run(device, q, k, v, meta, length, 2).float().cpu().numpy()
+    # one rounding of the output (2^-25: half of f16's subnormal step)
+    bound = ULP[dtype] * np.abs(expect) + 2.0 ** -16 * total + 2.0 ** -25
+    assert np.all(np.abs(got - expect) <= bound), float((np.abs(got - expect) / bound).max())
+
+
 @pytest.mark.parametrize("dim,groups,history", [(64, 4, 0), (128, 4, 700), (256, 2, 40)])
 def test_prefill_masked_keys_never_contribute(device, dim, groups, history):
     """A NaN and an infinity in V at one key: rows that do not see it are those of the finite V
