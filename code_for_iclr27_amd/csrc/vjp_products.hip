@@ -251,6 +251,17 @@ __global__ __launch_bounds__(kColumnThreads) void column_products_kernel(
       const prod_u32x2 hi = transposed(w_lane[t] + offset + 8 * (kColumnTile * 2));
       w[t] = prod_u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
+    // The copies of the last row stand for no row: their coefficients are zero, and as 0 * W is NaN
+    // for an infinite W they are cleared.
+    if (const int left = count - s * kColumnStage; left < kColumnStage) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = 4 * half + 8 * (i >> 1) + 2 * (i & 1);
+        const unsigned live_rows = k + 1 < left ? ~0u : k < left ? 0xffffu : 0u;
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) w[t][i] &= live_rows;
+      }
+    }
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) acc[t] = product(c, w[t], acc[t]);
     free = offset;

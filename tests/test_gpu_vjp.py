@@ -106,6 +106,22 @@ def test_row_hidden_gradients_several_rows(device, dtype, rows, vocab, dim):
     assert np.all(np.abs(got - expect) <= 2e-6 * scale)
 
 
+@pytest.mark.parametrize("rows,vocab,dim", [(3, 17, 128), (8, 63, 256), (5, 513, 512)])
+def test_row_hidden_gradients_infinite_weights(device, rows, vocab, dim):
+    """Infinities in the last weight rows (block and stage remainders) reach the gradients with
+    their sign in their own columns, as the f32 sum over the rows has it, and nothing else."""
+    model, _ = model_with_head(device, vocab, dim, seed=rows + 60)
+    w = model.get_output_embeddings().weight
+    w[vocab - 1, 3], w[vocab - 1, dim - 1], w[vocab - 2, 40] = float("inf"), float("-inf"), float("inf")
+    logits = torch.randn((rows, vocab), generator=torch.Generator().manual_seed(61)).to(device)
+    logits[:, 2] = 9.0  # the target of every row, a finite weight row
+    _, targets, competitors = vjp.row_margins(logits)
+    got = vjp.row_hidden_gradients(model, logits, targets, competitors, [1.0] * rows).cpu()
+    expect = torch.full((rows, dim), 0.0)
+    expect[:, 3], expect[:, dim - 1], expect[:, 40] = -float("inf"), float("inf"), -float("inf")
+    assert torch.equal(torch.where(torch.isfinite(got), torch.zeros(()), got), expect)
+
+
 def test_margins_given_and_argmax(device):
     rng = np.random.default_rng(3)
     logits = (rng.standard_normal((4, 128256)) * 3).astype(np.float32)
