@@ -191,12 +191,13 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
   const int end = bounds.key_end - begin > chunk ? begin + chunk : bounds.key_end;
 
   // Visible keys: this lane's row sees keys <= limit; the wave's rows see keys < wave_end, and
-  // those <= wave_limit are seen by all of them.
+  // those <= wave_limit are seen by all of them (with a zero scale no key counts as such).
   const int query = row_valid ? row / groups : 0;
   const int limit = row_valid ? query + bounds.shift : -1;
   const int wave_last = min(wave_row0 + kWaveRows, rows) - 1;
   const int wave_end = wave_row0 < rows ? min(end, wave_last / groups + bounds.shift + 1) : 0;
-  const int wave_limit = wave_row0 < rows ? wave_row0 / groups + bounds.shift : -1;
+  const int wave_limit =
+      wave_row0 < rows && a.scale != 0.0f ? wave_row0 / groups + bounds.shift : -1;
 
   const T* q_row = nullptr;
   {
@@ -206,13 +207,13 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
             static_cast<int64_t>(query) * a.q_query;
   }
   // B operand: k = half * D/2 + 8 * ks + [0, 8). The kernel works with a positive scale: a
-  // negative one goes into the queries' sign bits, and a zero one clears them.
+  // negative one goes into the queries' sign bits, and a zero one is multiplied into the scores as
+  // they are masked (then every stage's are), so that an infinite or NaN score becomes NaN.
   attn_u32x4 qop[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     qop[ks] = load16(q_row + half * (D / 2) + 8 * ks);
     if (a.scale < 0.0f) qop[ks] ^= 0x80008000u;
-    if (a.scale == 0.0f) qop[ks] = attn_u32x4{0u, 0u, 0u, 0u};
   }
 
   const __bf16* keys = static_cast<const __bf16*>(a.keys) + bounds.key0 * D;
@@ -236,6 +237,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
                                                   v_base + at, v_offset);
   };
 
+  const float unit = a.scale == 0.0f ? 0.0f : 1.0f;
   const float scale = a.scale == 0.0f ? 1.0f : __builtin_fabsf(a.scale);
   const float to_log2 = scale * kAttnLog2e;  // scores -> exponents of two
   float reference = kNegInf, sum = 0.0f;       // in exponents of two; the same in both halves
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
       top = kNegInf;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s[r] = key + tile_key(r, half) <= limit ? s[r] : kNegInf;
+        s[r] = key + tile_key(r, half) <= limit ? s[r] * unit : kNegInf;
         top = fmaxf(top, s[r]);
       }
     }

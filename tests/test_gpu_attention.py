@@ -177,30 +177,62 @@ def test_prefill_masked_keys_never_contribute(device, dim, groups, history):
     assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
 
 
+def through_the_abi(device, entry, q, k, v, meta, length, kv_heads, scale):
+    """lr_packed_attention, with a workspace of the size it asks for, or its allocation-free
+    variant: [batch, length, query heads * dim]."""
+    from code_for_iclr27_amd import _lib
+    tensors = [t.to(device) for t in (q, k, v)]
+    batch, heads, dim = q.shape[0], q.shape[1], q.shape[3]
+    groups, longest = heads // kv_heads, meta.max_seqlen_k
+    out = torch.full((batch, length, heads * dim), float("nan"), dtype=q.dtype, device=device)
+    size = _lib.load().lr_packed_attention_workspace_bytes(batch * kv_heads, groups, length,
+                                                           longest, dim)
+    workspace = torch.empty(max(size, 256), dtype=torch.uint8, device=device)
+    extra = [workspace.data_ptr(), workspace.numel()] if entry == "lr_packed_attention" else []
+    _lib.call(entry, tensors[0].data_ptr(), *tensors[0].stride()[:3], tensors[1].data_ptr(),
+              tensors[2].data_ptr(), k.shape[0], meta.cu_seqlens_k.data_ptr(), batch, kv_heads,
+              groups, length, dim, _lib.DTYPE_CODES[q.dtype], longest, scale, out.data_ptr(),
+              *extra, torch.cuda.current_stream().cuda_stream)
+    return out
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.125, 0.5, 2.0])
 def test_prefill_scales_through_the_abi(device, scale):
     """lr_packed_attention's scale is any number: zero (the mean of the visible values) and
     negative ones too. A larger scale has a larger relative rounding of the f32 exponents:
     2^-24 of logits up to 90 (scale 2 at d64) is 6e-6 of a probability, within the tolerance."""
-    from code_for_iclr27_amd import _lib
     length, kv_heads, groups, dim = 50, 2, 4, 64
     q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim, [50, 120], seed=19)
-    tensors = [t.to(device) for t in (q, k, v)]
-    out = torch.empty((1, length, kv_heads * groups, dim), dtype=q.dtype, device=device)
-    size = _lib.load().lr_packed_attention_workspace_bytes(kv_heads, groups, length, 120, dim)
-    workspace = torch.empty(max(size, 256), dtype=torch.uint8, device=device)
-    for entry, extra in (("lr_packed_attention", [workspace.data_ptr(), workspace.numel()]),
-                         ("lr_packed_attention_noalloc", [])):
-        out.fill_(float("nan"))
-        _lib.call(entry, tensors[0].data_ptr(), *tensors[0].stride()[:3], tensors[1].data_ptr(),
-                  tensors[2].data_ptr(), k.shape[0], meta.cu_seqlens_k.data_ptr(), 1, kv_heads,
-                  groups, length, dim, _lib.LR_DTYPE_BF16, 120, scale, out.data_ptr(), *extra,
-                  torch.cuda.current_stream().cuda_stream)
-        expect = oattention.packed_attention(q.float().numpy(), k.float().numpy(),
-                                             v.float().numpy(), cu, kv_heads, scale)
-        error = np.abs(out.view(1, length, -1).float().cpu().numpy() - expect)
+    expect = oattention.packed_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                         cu, kv_heads, scale)
+    for entry in ("lr_packed_attention", "lr_packed_attention_noalloc"):
+        out = through_the_abi(device, entry, q, k, v, meta, length, kv_heads, scale)
+        error = np.abs(out.float().cpu().numpy() - expect)
         bound = ULP[q.dtype] * np.abs(expect) + 1e-4 * float(v.float().abs().max())
         assert np.all(error <= bound)
+
+
+@pytest.mark.parametrize("groups,length,dim,keys", [
+    (4, 50, 64, [50, 120]),    # one-wave tiles
+    (8, 131, 128, [131] * 16), # tiles of four waves
+])
+def test_prefill_zero_scale_keeps_non_finite_scores(device, groups, length, dim, keys):
+    """Scale 0 times an infinite or NaN score is NaN: the rows of such a query, and those that see
+    an infinite key, are NaN; the others are the mean of their visible values as before."""
+    kv_heads = len(keys)
+    q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim, keys, seed=25)
+    clean = through_the_abi(device, "lr_packed_attention", q, k, v, meta, length, kv_heads, 0.0)
+    q[0, 1, 5, 3], q[0, 2, 7, dim - 1] = float("nan"), float("inf")
+    at = length - 9  # of the second segment
+    k[int(cu[1]) + keys[1] - length + at, 1] = float("-inf")
+    got = through_the_abi(device, "lr_packed_attention", q, k, v, meta, length, kv_heads, 0.0)
+    bad = torch.zeros((length, kv_heads * groups), dtype=torch.bool, device=device)
+    bad[5, 1], bad[7, 2], bad[at:, groups:2 * groups] = True, True, True
+    got, clean = (t.view(length, kv_heads * groups, dim) for t in (got, clean))
+    assert torch.isnan(got[bad]).all() and torch.isfinite(got[~bad]).all()
+    # a row that shares a wave with a bad one is taken again key by key: another order of the sums
+    bound = ULP[got.dtype] * clean.float().abs() * 2 + 2e-4 * float(v.float().abs().max())
+    assert torch.all((got.float() - clean.float()).abs()[~bad] <= bound[~bad])
 
 
 def test_strided_queries_as_the_reference_builds_them(device):
