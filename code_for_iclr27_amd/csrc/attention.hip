@@ -430,13 +430,16 @@ bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_k
   return dim == 64 || !few_rows || max_keys <= 128 || max_keys > 40000 / segments;
 }
 
-// The prefill kernel's plan. Its partial states stay within the allocation-free entry point's
-// array for every call that entry point accepts (its limit is the split-key plan's bytes, below),
-// and within 32 MiB otherwise.
+// The prefill kernel's plan. Calls whose segments fit one block of the split-key kernel's keys need
+// no workspace, so their keys are not split here either. Other partial states stay within the
+// allocation-free entry point's array for every call that entry point accepts (its limit is the
+// split-key plan's bytes, below), and within 32 MiB otherwise.
 AttnTilePlan plan_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys,
                         int64_t dim) {
   const size_t blocks = workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim);
-  const size_t most = blocks <= kAttentionScratchBytes ? kAttentionScratchBytes : size_t{32} << 20;
+  const size_t most = blocks == 0                        ? 0
+                      : blocks <= kAttentionScratchBytes ? kAttentionScratchBytes
+                                                         : size_t{32} << 20;
   return plan_attention_tiles(segments, groups, length, max_keys, dim, static_cast<int64_t>(most));
 }
 

@@ -467,9 +467,10 @@ int lr_history_append(const void* const* layer_queries, int64_t layers, int64_t 
  * with no visible key is zero. out is [batch, length, kv_heads*groups, dim] contiguous, of the
  * input dtype (LR_DTYPE_BF16 or LR_DTYPE_F16); dim in {64, 128, 256}. max_keys bounds every
  * segment's key count (keys past it are not read). workspace: device scratch of at least
- * lr_packed_attention_workspace_bytes(...) bytes (0 when no segment's keys are split over
- * workgroups), 256-byte aligned, no initial contents required; calls that overlap in time need
- * their own. Two launches when they are split (key blocks, then their merge). */
+ * lr_packed_attention_workspace_bytes(...) bytes, 256-byte aligned, no initial contents required;
+ * calls that overlap in time need their own. 0 bytes when every segment fits one block of keys
+ * (max_keys, with a pending row, up to 384, 192, 128 at dim 64, 128, 256), and wherever the keys
+ * are not split over workgroups; two launches when they are (key blocks, then their merge). */
 size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t groups, int64_t length,
                                            int64_t max_keys, int64_t dim);
 int lr_packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head_stride,

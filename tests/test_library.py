@@ -69,6 +69,18 @@ def test_noalloc_attention_size_check_needs_no_gpu():
     assert status == 1 and "holds at most 16777216 bytes" in _lib.last_error()
 
 
+@pytest.mark.parametrize("dim,keys", [(64, 384), (128, 192), (256, 128)])
+def test_attention_over_one_key_block_needs_no_workspace(dim, keys):
+    """Whatever kernel runs, a call whose segments fit one block of keys takes a NULL workspace
+    (and leaves the allocation-free entry point's shared array alone)."""
+    size = _lib.load().lr_packed_attention_workspace_bytes
+    for segments in (1, 2, 8, 64, 500):
+        for groups in (1, 3, 4, 8):
+            for length in (1, 2, 5, 8, 32, 100, 384):
+                for longest in (1, 33, 64, keys - 65, keys - 1, keys):
+                    assert size(segments, groups, length, longest, dim) == 0, (segments, longest)
+
+
 def test_stream_copy_checks_size_and_alignment_on_host():
     library = _lib.load()
     assert library.lr_stream_copy(None, None, 0, None) == 0
