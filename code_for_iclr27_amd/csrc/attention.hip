@@ -252,6 +252,33 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
         for (int e = 0; e < 8; ++e) acc[r][e] = __builtin_fmaf(p, v[e], acc[r][e]);
       }
     }
+    // A masked key's p is 0, and 0 * V is NaN for a non-finite V: a wave with a non-finite sum takes
+    // its rows again, over the keys that each of them sees. (Every row of a decode call sees all.)
+    if (a.length > 1) {
+      float poison = 0.f;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) poison = __builtin_fmaf(acc[r][e], 0.f, poison);
+      if (__any(poison != poison)) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
+#pragma unroll 1
+        for (int key = kg; key < nk; key += KPI) {
+          float v[8];
+          unpack8<T>(load16(vbase + key * D + 8 * c), v);
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            if (key > static_cast<int>(query_of(a, row0 + r)) + keys.shift - kb) continue;
+            const float p = probs[wave][key][r];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[r][e] = __builtin_fmaf(p, v[e], acc[r][e]);
+          }
+        }
+      }
+    }
     // Sum the KPI lane groups (lanes c, c + LPK, ... hold the same elements).
 #pragma unroll
     for (int r = 0; r < R; ++r)

@@ -177,6 +177,27 @@ def test_prefill_masked_keys_never_contribute(device, dim, groups, history):
     assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
 
 
+@pytest.mark.parametrize("dim,groups,length,history", [(64, 1, 3, 200), (128, 1, 5, 720),
+                                                       (128, 4, 8, 30), (256, 6, 8, 200)])
+def test_few_queries_masked_keys_never_contribute(device, dim, groups, length, history):
+    """The same where a few query rows on a cached prefix run the split-key kernel."""
+    kv_heads = 2
+    q, k, v, cu, meta = make(device, 1, kv_heads, groups, length, dim,
+                             [history + length] * kv_heads, seed=28)
+    finite = run(device, q, k, v, meta, length, kv_heads)
+    check(finite, q, k, v, cu, kv_heads)
+    bad = v.clone()
+    bad[history + length - 1, 3], bad[history + length - 1, dim - 1] = float("nan"), float("inf")
+    got = run(device, q, k, bad, meta, length, kv_heads).view(length, kv_heads, groups, dim)
+    finite = finite.view(length, kv_heads, groups, dim)
+    columns = torch.tensor([3, dim - 1], device=device)
+    assert not torch.isfinite(got[-1, 0][..., columns]).any()
+    changed = torch.zeros_like(got, dtype=torch.bool)
+    changed[-1, 0] = torch.isin(torch.arange(dim, device=device), columns)
+    bound = ULP[got.dtype] * finite.float().abs() * 2 + 2e-4 * float(v.float().abs().max())
+    assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
+
+
 def through_the_abi(device, entry, q, k, v, meta, length, kv_heads, scale):
     """lr_packed_attention, with a workspace of the size it asks for, or its allocation-free
     variant: [batch, length, query heads * dim]."""
