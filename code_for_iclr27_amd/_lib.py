@@ -85,6 +85,7 @@ SIGNATURES = {
     "lr_copy_words": [_P, _P, _I64, _P],
     "lr_stream_copy": [_P, _P, _I64, _P],
     "lr_packed_attention_workspace_bytes": [_I64, _I64, _I64, _I64, _I64],
+    "lr_packed_attention_plan": [_I64, _I64, _I64, _I64, _I64, _I, _P],
     "lr_packed_attention": [_P, _I64, _I64, _I64, _P, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64,
                             _I, _I64, _F, _P, _P, _SZ, _P],
     "lr_packed_attention_pending_workspace_bytes": [_I64, _I64, _I64, _I64],

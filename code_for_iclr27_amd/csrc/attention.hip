@@ -445,18 +445,6 @@ size_t workspace_bytes(const AttnPlan& p, int64_t dim) {
   return static_cast<size_t>(slots) * static_cast<size_t>(dim + 2) * 4;
 }
 
-// Whether a call runs the prefill kernel (attention_tile.hip). The split-key kernel stays for
-// decode, and for the few rows a 32-row tile would leave mostly empty: up to 32 rows on a cached
-// prefix (d128, G4: 2 queries on 500 keys 10.9 us against 12.5, 8 queries on 4000 keys 23.2
-// against 25.0), while the segments' keys fit one round of its blocks (3 x 8 segments of 2,861
-// keys, 8 queries: 35.1 against 23.1 us). At d64 the tiles are already ahead (2 queries on 500
-// keys 9.1 against 11.5 us, 8 on 4000 14.9 against 32.8).
-bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys, int64_t dim) {
-  if (length <= 1) return false;
-  const bool few_rows = length * groups <= 32;
-  return dim == 64 || !few_rows || max_keys <= 128 || max_keys > 40000 / segments;
-}
-
 // The prefill kernel's plan. Calls whose segments fit one block of the split-key kernel's keys need
 // no workspace, so their keys are not split here either. Other partial states stay within the
 // allocation-free entry point's array for every call that entry point accepts (its limit is the
@@ -468,6 +456,40 @@ AttnTilePlan plan_tiles(int64_t segments, int64_t groups, int64_t length, int64_
                       : blocks <= kAttentionScratchBytes ? kAttentionScratchBytes
                                                          : size_t{32} << 20;
   return plan_attention_tiles(segments, groups, length, max_keys, dim, static_cast<int64_t>(most));
+}
+
+// Whether a call of several queries runs the prefill kernel (attention_tile.hip): where its estimate
+// is the lower one. A call of the split-key kernel takes `call` us, less for few keys or rows; its
+// blocks add up on a CU once there are more than alone / block of them, and a split call pays the
+// merge and its partial states. The prefill plan's own estimate is scaled (an f16 stage takes
+// longer). Fitted to 3,600 shapes (each head dimension, 2 to 64 segments, 1 to 8 groups, 2 to 256
+// queries, 2 to 4,000 keys) timed with both kernels: the choice is 0.1% to 0.8% above the better one
+// on average, by dimension and type. Both sides, us, split-key and tiles: 4 segments, G6, 8 queries
+// on 200 keys at d256 10.8 and 14.7; 8 segments, G4, 32 queries on 300 at d64, f16, 9.9 and 15.4;
+// 24 segments, G4, 2 queries on 4,000 at d128 27.4 and 20.4.
+struct SplitKeyTimes {
+  double call, alone, block, small_block, merge, megabyte;
+};
+bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_keys, int64_t dim,
+                 int dtype) {
+  if (length <= 1) return false;
+  const SplitKeyTimes us = dim == 64    ? SplitKeyTimes{7.4, 1.2, 2.4, 0.6, 0.4, 2.5}
+                           : dim == 128 ? SplitKeyTimes{7.5, 0.7, 2.2, 0.75, 1.3, 1.3}
+                                        : SplitKeyTimes{7.9, 0.5, 3.7, 1.75, 2.0, 0.6};
+  const AttnPlan plan = plan_attention(segments, groups, length, max_keys, dim);
+  const double load = static_cast<double>(plan.units) * static_cast<double>(plan.splits) / 256.0 *
+                      (plan.wave_keys == kSmallWaveKeys ? us.small_block : us.block);
+  const double split_key =
+      us.call - (plan.rows_per_tile == 4 ? 1.0 : 0.0) -
+      0.04 * static_cast<double>(std::max<int64_t>(0, 64 - max_keys)) + std::max(us.alone, load) +
+      (plan.splits > 1 ? us.merge + us.megabyte * 1e-6 * static_cast<double>(workspace_bytes(plan, dim))
+                       : 0.0);
+  const bool f16 = dtype == LR_DTYPE_F16;
+  const double estimate = plan_tiles(segments, groups, length, max_keys, dim).us;
+  const double tiles = dim == 64    ? (f16 ? 3.1 + 1.59 * estimate : 3.2 + 1.23 * estimate)
+                       : dim == 128 ? (f16 ? 3.5 + 1.48 * estimate : 2.9 + 1.30 * estimate)
+                                    : (f16 ? 5.3 + 1.44 * estimate : 4.2 + 1.22 * estimate);
+  return tiles < split_key;
 }
 
 template <typename T, int D, int R, int CH>
@@ -525,9 +547,32 @@ extern "C" size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t 
                                                       int64_t length, int64_t max_keys,
                                                       int64_t dim) {
   if (segments <= 0 || groups <= 0 || length <= 0 || max_keys < 0 || dim <= 0) return 0;
-  if (takes_tiles(segments, groups, length, max_keys, dim))
-    return attention_tiles_bytes(plan_tiles(segments, groups, length, max_keys, dim), dim);
-  return workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim);
+  // what either type needs: which kernel runs depends on it
+  size_t bytes = 0;
+  for (const int dtype : {LR_DTYPE_BF16, LR_DTYPE_F16})
+    bytes = std::max(bytes,
+                     takes_tiles(segments, groups, length, max_keys, dim, dtype)
+                         ? attention_tiles_bytes(plan_tiles(segments, groups, length, max_keys, dim), dim)
+                         : workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim));
+  return bytes;
+}
+
+extern "C" int lr_packed_attention_plan(int64_t segments, int64_t groups, int64_t length,
+                                        int64_t max_keys, int64_t dim, int dtype, int64_t* plan) {
+  clear_error();
+  LR_REQUIRE(dim == 64 || dim == 128 || dim == 256, "Head dimension must be 64, 128 or 256");
+  LR_REQUIRE(segments > 0 && groups > 0 && length > 0 && max_keys >= 0 && plan,
+             "Empty attention dimensions");
+  if (takes_tiles(segments, groups, length, max_keys, dim, dtype)) {
+    const AttnTilePlan tiles = plan_tiles(segments, groups, length, max_keys, dim);
+    plan[0] = tiles.rows;
+    plan[1] = tiles.splits;
+  } else {
+    const AttnPlan blocks = plan_attention(segments, groups, length, max_keys, dim);
+    plan[0] = blocks.rows_per_tile;
+    plan[1] = blocks.splits;
+  }
+  return LR_OK;
 }
 
 namespace lr {
@@ -563,7 +608,7 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
   const int64_t segments = batch * kv_heads;
   if (pending_keys != nullptr) ++max_keys;  // every segment's pending row
   const AttnPlan plan = plan_attention(segments, groups, length, max_keys, dim);
-  const bool use_tiles = takes_tiles(segments, groups, length, max_keys, dim);
+  const bool use_tiles = takes_tiles(segments, groups, length, max_keys, dim, dtype);
   AttnTilePlan tile_plan{};
   if (use_tiles) tile_plan = plan_tiles(segments, groups, length, max_keys, dim);
   const size_t needed =

@@ -513,7 +513,11 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
 }
 
 // Second launch of a split call: a thread folds one (row, 8 columns) slice of a tile over the
-// key chunks, in chunk order. References are exponents of two.
+// key chunks, in chunk order, a round of chunks' states loaded together: a memory round trip a
+// round. (One a chunk: 16 queries on 4,000 keys, 8 segments, G4, d64 28.7 us against 15.) References
+// are exponents of two.
+constexpr int kMergeRound = 8;
+
 template <typename T, int D, int ROWS>
 __global__ __launch_bounds__(kAttnThreads) void prefill_merge_kernel(AttnArgs a, int chunk) {
   constexpr int LPR = D / 8, kBlocks = ROWS * LPR / kAttnThreads;
@@ -530,22 +534,31 @@ __global__ __launch_bounds__(kAttnThreads) void prefill_merge_kernel(AttnArgs a,
   if (needed <= 1 || row0 + r >= rows) return;
   float top = kNegInf, sum = 0.0f, o[8] = {};
   const int64_t first = static_cast<int64_t>(unit) * a.splits * ROWS + r;
-  for (int k = 0; k < needed; ++k) {
-    const int64_t at = first + static_cast<int64_t>(k) * ROWS;
-    const float m = a.part_ml[at * 2], l = a.part_ml[at * 2 + 1];
-    const attn_f32x4 x = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * c);
-    const attn_f32x4 y = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * c + 4);
-    if (m == kNegInf) continue;
-    const float higher = fmaxf(top, m);
-    const float ws = top == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(top - higher);
-    const float wo = __builtin_amdgcn_exp2f(m - higher);
-    sum = __builtin_fmaf(wo, l, sum * ws);
+  for (int k0 = 0; k0 < needed; k0 += kMergeRound) {
+    float m[kMergeRound], l[kMergeRound];
+    attn_f32x4 x[kMergeRound], y[kMergeRound];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[e] = __builtin_fmaf(wo, x[e], o[e] * ws);
-      o[4 + e] = __builtin_fmaf(wo, y[e], o[4 + e] * ws);
+    for (int i = 0; i < kMergeRound; ++i) {
+      const int64_t at = first + static_cast<int64_t>(min(k0 + i, needed - 1)) * ROWS;
+      m[i] = k0 + i < needed ? a.part_ml[at * 2] : kNegInf;
+      l[i] = a.part_ml[at * 2 + 1];
+      x[i] = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * c);
+      y[i] = *reinterpret_cast<const attn_f32x4*>(a.part_o + at * D + 8 * c + 4);
     }
-    top = higher;
+#pragma unroll
+    for (int i = 0; i < kMergeRound; ++i) {
+      if (m[i] == kNegInf) continue;
+      const float higher = fmaxf(top, m[i]);
+      const float ws = top == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(top - higher);
+      const float wo = __builtin_amdgcn_exp2f(m[i] - higher);
+      sum = __builtin_fmaf(wo, l[i], sum * ws);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[e] = __builtin_fmaf(wo, x[i][e], o[e] * ws);
+        o[4 + e] = __builtin_fmaf(wo, y[i][e], o[4 + e] * ws);
+      }
+      top = higher;
+    }
   }
   const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
 #pragma unroll
@@ -595,8 +608,8 @@ int launch_tile_dim(const AttnArgs& args, const AttnTilePlan& plan, int64_t dim,
 // once there are more than 1024 * alone / wave. Splitting the keys costs the merge launch and its
 // partial states. Fitted to 129 shapes (every head dimension, 2 to 2048 queries on 0 to 4096
 // cached keys, 1 to 8 groups, each at up to 20 tile and chunk choices): the choice is 2.6% above
-// the best one on average. One tile and no chunks, by contrast: 8192 new queries the same 880 us,
-// 32 queries on 4000 keys 126 us instead of 30 (8B shape).
+// the best one on average. One tile and no chunks, by contrast: 8192 new queries the same 850 us,
+// 32 queries on 4000 keys 126 us instead of 22 (8B shape).
 struct StageTimes {
   double alone, tile, wave;
 };
@@ -625,7 +638,7 @@ AttnTilePlan plan_attention_tiles(int64_t segments, int64_t groups, int64_t leng
                           (splits > 1 ? 2.0 + 0.4e-6 * bytes : 0.0);
       if (best.splits == 0 || time < least) {
         least = time;
-        best = {segments, rows, tiles, splits, std::min<int64_t>(per * kStageKeys, INT32_MAX)};
+        best = {segments, rows, tiles, splits, std::min<int64_t>(per * kStageKeys, INT32_MAX), time};
       }
     }
   }

@@ -7,6 +7,7 @@ namespace lr {
 
 struct AttnTilePlan {
   int64_t segments, rows, tiles, splits, chunk;  // rows of a tile, keys of one split
+  double us;  // the estimate it was chosen by (bf16, launches not counted)
 };
 
 // `scratch_bytes` bounds the partial states of a call that splits its keys.

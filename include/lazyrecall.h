@@ -470,9 +470,14 @@ int lr_history_append(const void* const* layer_queries, int64_t layers, int64_t 
  * lr_packed_attention_workspace_bytes(...) bytes, 256-byte aligned, no initial contents required;
  * calls that overlap in time need their own. 0 bytes when every segment fits one block of keys
  * (max_keys, with a pending row, up to 384, 192, 128 at dim 64, 128, 256), and wherever the keys
- * are not split over workgroups; two launches when they are (key blocks, then their merge). */
+ * are not split over workgroups; two launches when they are (key blocks, then their merge). The
+ * size holds for both types. */
 size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t groups, int64_t length,
                                            int64_t max_keys, int64_t dim);
+/* How a call of these sizes runs (host only): plan[0] query rows of a tile (4 or 8: the split-key
+ * kernel, 32 or 128: the prefill kernel), plan[1] the parts its keys are split into. */
+int lr_packed_attention_plan(int64_t segments, int64_t groups, int64_t length, int64_t max_keys,
+                             int64_t dim, int dtype, int64_t* plan);
 int lr_packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head_stride,
                         int64_t q_query_stride, const void* keys, const void* values,
                         int64_t key_rows, const int32_t* cu_seqlens_k, int64_t batch,

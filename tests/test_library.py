@@ -81,6 +81,35 @@ def test_attention_over_one_key_block_needs_no_workspace(dim, keys):
                     assert size(segments, groups, length, longest, dim) == 0, (segments, longest)
 
 
+def attention_plan(segments, groups, length, keys, dim, dtype=_lib.LR_DTYPE_BF16):
+    plan = np.zeros(2, np.int64)
+    assert _lib.load().lr_packed_attention_plan(segments, groups, length, keys, dim, dtype,
+                                                plan.ctypes.data) == 0
+    return plan.tolist()
+
+
+def test_attention_runs_the_faster_kernel_where_they_differ_much():
+    """Shapes at which one of the kernels measured at least a twentieth longer, most of them far."""
+    f16 = _lib.LR_DTYPE_F16
+    split_key = [(4, 6, 8, 208, 256), (4, 6, 16, 516, 256), (4, 6, 8, 1008, 256), (8, 4, 2, 302, 64, f16),
+                 (8, 4, 32, 332, 64, f16), (4, 6, 8, 308, 256, f16), (8, 4, 1, 9000, 128)]
+    tiles = [(24, 4, 2, 4002, 128), (24, 4, 4, 4004, 128), (8, 4, 8192, 8192, 128), (8, 4, 333, 333, 64), (8, 4, 333, 333, 64, f16),
+             (4, 6, 1000, 5000, 256), (4, 6, 1000, 5000, 256, f16), (8, 4, 8, 4008, 64),
+             (24, 4, 8, 2861, 128), (8, 4, 32, 100, 64), (8, 4, 128, 1128, 128)]
+    assert all(attention_plan(*shape)[0] <= 8 for shape in split_key)
+    assert all(attention_plan(*shape)[0] >= 32 for shape in tiles)
+
+
+def test_attention_workspace_covers_both_types():
+    size = _lib.load().lr_packed_attention_workspace_bytes
+    for shape in [(8, 4, 2, 900, 64), (8, 4, 16, 4016, 128), (4, 6, 32, 532, 256), (4, 6, 32, 132, 256)]:
+        segments, groups, length, _, dim = shape
+        for dtype in (_lib.LR_DTYPE_BF16, _lib.LR_DTYPE_F16):
+            rows, splits = attention_plan(*shape, dtype)
+            slots = segments * -(-length * groups // rows) * splits * rows
+            assert size(*shape) >= (slots * (dim + 2) * 4 if splits > 1 else 0)
+
+
 def test_stream_copy_checks_size_and_alignment_on_host():
     library = _lib.load()
     assert library.lr_stream_copy(None, None, 0, None) == 0
