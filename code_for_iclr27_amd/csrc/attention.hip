@@ -465,7 +465,7 @@ AttnTilePlan plan_tiles(int64_t segments, int64_t groups, int64_t length, int64_
 // longer). Fitted to 3,600 shapes (each head dimension, 2 to 64 segments, 1 to 8 groups, 2 to 256
 // queries, 2 to 4,000 keys) timed with both kernels: the choice is 0.1% to 0.8% above the better one
 // on average, by dimension and type. Both sides, us, split-key and tiles: 4 segments, G6, 8 queries
-// on 200 keys at d256 10.8 and 14.7; 8 segments, G4, 32 queries on 300 at d64, f16, 9.9 and 15.4;
+// on 200 keys at d256 10.8 and 14.7; 8 segments, G4, 32 queries on 300 at d64, f16, 9.9 and 12.5;
 // 24 segments, G4, 2 queries on 4,000 at d128 27.4 and 20.4.
 struct SplitKeyTimes {
   double call, alone, block, small_block, merge, megabyte;
@@ -486,9 +486,9 @@ bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_k
                        : 0.0);
   const bool f16 = dtype == LR_DTYPE_F16;
   const double estimate = plan_tiles(segments, groups, length, max_keys, dim).us;
-  const double tiles = dim == 64    ? (f16 ? 3.1 + 1.59 * estimate : 3.2 + 1.23 * estimate)
-                       : dim == 128 ? (f16 ? 3.5 + 1.48 * estimate : 2.9 + 1.30 * estimate)
-                                    : (f16 ? 5.3 + 1.44 * estimate : 4.2 + 1.22 * estimate);
+  const double tiles = dim == 64    ? (f16 ? 3.2 + 1.39 * estimate : 3.2 + 1.23 * estimate)
+                       : dim == 128 ? (f16 ? 3.4 + 1.42 * estimate : 2.9 + 1.30 * estimate)
+                                    : (f16 ? 5.1 + 1.44 * estimate : 4.2 + 1.22 * estimate);
   return tiles < split_key;
 }
 

@@ -1,39 +1,40 @@
 // Prefill attention: packed attention (attention.hip states the layout and the causal rule) for
 // calls with many query rows, where both products are matrix work.
 //
-// A workgroup of four waves owns 128 query rows (row = i*G + g) of one segment, 32 per wave, and
-// streams the segment's keys in stages of 64 (d256: 32) rows of K and V, copied straight to LDS
-// and double-buffered. Per 32 keys a wave forms S^T = K Q^T on v_mfma_f32_32x32x16 (a lane holds
-// one query's scores of 16 keys), takes the exponentials against a running reference, and
-// accumulates O^T += V^T P^T. The contraction's key order is free, so the probabilities stay
-// where S^T left them: a lane's accumulators 8k .. 8k+7 are the B operand of 16 keys, and the A
-// operand reads the same keys' V columns with the transposing LDS load (ds_read_b64_tr_b16: 4
-// keys of one column per lane).
+// A workgroup of four waves owns 128 query rows (row = i*G + g) of one segment, 32 per wave, or one
+// of a single wave 32 rows (short calls, where 128-row tiles would leave CUs idle). It streams the
+// segment's keys in stages of 32 rows of K and V, copied straight to LDS and double-buffered. In a
+// stage a wave forms S^T = K Q^T on v_mfma_f32_32x32x16 (a lane holds one query's scores of 16
+// keys), takes the exponentials against a running reference, and accumulates O^T += V^T P^T. The
+// contraction's key order is free, so the probabilities stay where S^T left them: a lane's
+// accumulators 8k .. 8k+7 are the B operand of 16 keys, and the A operand reads the same keys' V
+// columns with the transposing LDS load (ds_read_b64_tr_b16: 4 keys of one column per lane).
 //
 // Precision. P is f32 and stays f32: it enters the 16-bit MFMA as a sum of 16-bit pieces whose
 // products with V are exact in f32. bf16: three pieces by truncation, 3 x 8 bits = the whole
 // 24-bit significand. f16: pieces by rounding. With P scaled by 2^11 two of them hold 11 + 11 bits
 // and a sign, but nothing below 2^-25 (f16's subnormals), which is 2^-12 of P = 2^-24. So what they
-// leave goes, 2^24 times larger, into two more pieces (the tails) whose products are summed apart
-// and added to the output once a stage. The four are within 2^-60 of P (all of its bits down to
-// 2^-36 of the reference): n keys are within 2^-44 n of the sum with f32 P, for any f16 V, against
-// output steps of 2^-24 and more.
+// leave goes, 2^24 times larger, into two more pieces (the tails), whose products are summed in
+// accumulators of their own, or, where those would cost occupancy, a stage at a time. The four are
+// within 2^-60 of P (all of its bits down to 2^-36 of the reference): n keys are within 2^-44 n of
+// the sum with f32 P, for any f16 V, against output steps of 2^-24 and more.
 //
 // The reference of a row's exponentials only moves when the row's maximum has outgrown it by
 // 2^kSlack (the accumulators are rescaled then, seldom after the first stages); sums and products
 // are f32 throughout, so a reference below the maximum loses nothing.
 //
-// What bounds it: the matrix cores, at 8 MFMAs of scores and 24 of products (bf16) per 32 keys
-// and wave at d128, with about 170 vector instructions beside them. Measured (us, against the
+// What bounds it: the matrix cores, at 8 MFMAs of scores and 24 of products (bf16; f16 32) per 32
+// keys and wave at d128, with about 170 vector instructions beside them. Measured (us, against the
 // split-key kernel of attention.hip, whose 8-row tiles read every K and V row once each and
-// multiply P*V on the VALU): 8192 queries of the 8B shape 883 against 10,878 (1.25 PFLOP/s of
+// multiply P*V on the VALU): 8192 queries of the 8B shape 868 against 10,878 (1.25 PFLOP/s of
 // MFMA work), 1000 queries on 4,000 cached keys at d256, G6, 233 against 2,115. f16: 333 queries
-// at d64 15.4 against 24.3, 8192 at d128 1,140 against 10,768 (two pieces without the tails, which
-// lose the small P, 10.6 and 772; V as two bf16 pieces, six products, 15.3 and 1,717). Three waves
-// per SIMD (168 VGPRs, a few spills outside the loop) beat two without spills at d <= 128: 890
-// against 928 (f16 at d128, with the tails' accumulators, holds two). d256 holds one wave per SIMD (its
-// accumulators alone take 128 VGPRs), so its stream is laid out by hand: 233 against 285.
-// Stages of 64 keys, a third stage buffer, 32-row tiles for long prompts: no faster or slower.
+// at d64 13.4 against 24.3, 8192 at d128 1,120 against 10,768 (two pieces without the tails, which
+// lose the small P, 10.6 and 772; V as two bf16 pieces and six products 15.3 and 1,717; every
+// tail a stage at a time 14.6 and 1,139). Three waves per SIMD (168 VGPRs, a few spills outside the
+// loop) beat two without spills at d <= 128: 890 against 928; f16 at d128 holds two. d256 holds one
+// wave per SIMD (its accumulators alone take 128 VGPRs), so its stream is laid out by hand: 233
+// against 285. Stages of 64 keys, a third stage buffer, 32-row tiles for long prompts: no faster or
+// slower.
 //
 // A masked key never contributes: scores past a query's limit become -inf. Their P is 0, and as
 // 0 * V is NaN for a non-finite V, a wave that ends with a non-finite accumulator recomputes its
@@ -63,6 +64,7 @@ constexpr int kBuffers = 2;     // K and V stages in LDS
 template <typename T> struct TileVec;
 template <> struct TileVec<__bf16> {
   static constexpr int kPieces = 3, kTails = 0;
+  static constexpr float kTailScale = 1.0f;
   static constexpr float kRaise = 0.0f;
   static __device__ __forceinline__ tile_f32x16 mfma(attn_u32x4 a, attn_u32x4 b, tile_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(attn_bf16x8, a),
@@ -97,11 +99,15 @@ template <> struct TileVec<_Float16> {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (i == kPieces) x *= kTailScale, y *= kTailScale;
-      const half2 part = {static_cast<_Float16>(x), static_cast<_Float16>(y)};
+      half2 part = {static_cast<_Float16>(x), static_cast<_Float16>(y)};
+      // Hidden from the compiler, which would round each half once more for the differences, and not
+      // take them in one instruction of mixed types each.
+      float minus = -1.0f;
+      asm("" : "+v"(part), "+s"(minus));
       piece[i][w] = __builtin_bit_cast(unsigned, part);
       if (i == 3) break;
-      x -= static_cast<float>(part[0]);
-      y -= static_cast<float>(part[1]);
+      x = __builtin_fmaf(static_cast<float>(part[0]), minus, x);
+      y = __builtin_fmaf(static_cast<float>(part[1]), minus, y);
     }
   }
 };
@@ -154,6 +160,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
   constexpr int KS = D / 16;  // MFMA k-steps over the head dimension
   constexpr int DT = D / 32;  // 32-column tiles of the output
   constexpr bool kLaidOut = D == 256 || WAVES == 1;
+  // Accumulators of the tails' products, or (0) none kept: at d128 they would leave a four-wave
+  // tile one wave a SIMD and at d256 spill, so each stage's go into the output at once there.
+  constexpr int kKept = Vec::kTails == 0 || D == 256 || (D == 128 && !kLaidOut) ? 0 : DT;
   constexpr int kThreads = 64 * WAVES, kRows = kWaveRows * WAVES;
   __shared__ __align__(16) uint16_t k_lds[kBuffers][KEYS * D];
   __shared__ __align__(16) uint16_t v_lds[kBuffers][KEYS * D];
@@ -246,6 +255,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) out[dt][r] = 0.0f;
+  tile_f32x16 tail[kKept > 0 ? kKept : 1];
+#pragma unroll
+  for (int dt = 0; dt < kKept; ++dt) tail[dt] = out[dt];
 
   // The lane's transposed reads: row 4 * half + (lane % 16) / 4 of an 8-row group, columns
   // 16 * (lane / 16 % 2) + 4 * (lane % 4) .. + 3 of a 32-column tile (chunk dt * 4 + v_chunk).
@@ -289,7 +301,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[dt][r] *= factor;
+        for (int r = 0; r < 16; ++r) {
+          out[dt][r] *= factor;
+          if constexpr (kKept > 0) tail[dt][r] *= factor;
+        }
       reference = raised;
     }
   };
@@ -349,26 +364,27 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
           Vec::split(p[e], p[e + 1], piece[e / 8], (e / 2) % 4);
         }
       };
-      constexpr int kProducts = Vec::kPieces * DT;
+      constexpr int kProducts = Vec::kPieces * DT + Vec::kTails * kKept;
       float top = kNegInf;
       auto product = [&](int k, int i) {
-        out[i % DT] = Vec::mfma(v_op[k][i % DT], piece[k][i / DT], out[i % DT]);
+        tile_f32x16& sums = i < Vec::kPieces * DT ? out[i % DT] : tail[kKept > 0 ? i % DT : 0];
+        sums = Vec::mfma(v_op[k][i % DT], piece[k][i / DT], sums);
       };
-      // The tails' products with all 32 keys, by column tiles.
+      // The tails' products with all 32 keys where no accumulators are kept, by column tiles.
       auto add_tails = [&]() {
-        if constexpr (Vec::kTails > 0) {
+        if constexpr (Vec::kTails > 0 && kKept == 0) {
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
-            tile_f32x16 tail;
+            tile_f32x16 rest;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) tail[r] = 0.0f;
+            for (int r = 0; r < 16; ++r) rest[r] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 2 * Vec::kTails; ++i)
-              tail = Vec::mfma(v_op[i / Vec::kTails][dt],
-                               piece[i / Vec::kTails][Vec::kPieces + i % Vec::kTails], tail);
+              rest = Vec::mfma(v_op[i / Vec::kTails][dt],
+                               piece[i / Vec::kTails][Vec::kPieces + i % Vec::kTails], rest);
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-              out[dt][r] = __builtin_fmaf(tail[r], 1.0f / Vec::kTailScale, out[dt][r]);
+              out[dt][r] = __builtin_fmaf(rest[r], 1.0f / Vec::kTailScale, out[dt][r]);
           }
         }
       };
@@ -433,6 +449,11 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(
     here = ahead, ahead = done;
   }
   sum += __shfl_xor(sum, 32);
+#pragma unroll
+  for (int dt = 0; dt < kKept; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      out[dt][r] = __builtin_fmaf(tail[dt][r], 1.0f / Vec::kTailScale, out[dt][r]);
 
   float poison = 0.0f;  // NaN if any accumulator is not finite
 #pragma unroll
