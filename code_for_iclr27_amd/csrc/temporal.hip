@@ -8,6 +8,7 @@
 // within a wave, LDS across waves), so sums may differ from the reference's 256-lane tree in
 // the last bits.
 
+#include <algorithm>
 #include <cmath>
 
 #include "lr_common.hpp"
@@ -361,6 +362,8 @@ __global__ __launch_bounds__(256) void decision_risk_kernel(
   }
 }
 
+constexpr int64_t kLaunchThreads = int64_t{1} << 32;
+
 template <typename T>
 int launch_probabilities(const void* logits, const float* projected, const int64_t* qpos,
                          const float* kpos, int64_t window, int64_t groups, int64_t length,
@@ -376,6 +379,8 @@ int launch_probabilities(const void* logits, const float* projected, const int64
   if (length <= 256 * 4) launch(probabilities_kernel<T, 256, 4>, 256);
   else if (length <= 256 * 9) launch(probabilities_kernel<T, 256, 9>, 256);
   else if (length <= 256 * 16) launch(probabilities_kernel<T, 256, 16>, 256);
+  // a launch has fewer than 2^32 threads: past 2^22 rows the blocks stay narrow
+  else if (rows >= kLaunchThreads / 1024) launch(probabilities_kernel<T, 256, 0>, 256);
   else if (length <= 1024 * 16) launch(probabilities_kernel<T, 1024, 16>, 1024);
   else launch(probabilities_kernel<T, 1024, 0>, 1024);
   return check_launch("temporal_probabilities");
@@ -428,13 +433,17 @@ int risk_scores(const float* probabilities, const float* output_projection, cons
   LR_REQUIRE(probabilities && output_projection && projected && margin && result,
              "Expected contiguous CUDA tensor");
   const int64_t count = last - first;
-  const int64_t blocks = ceil_div(count, kRiskCandidates);
   const hipStream_t s = as_stream(stream);
   const float eps = static_cast<float>(epsilon);
+  // As many candidates a launch as its threads (fewer than 2^32) allow.
+  constexpr int64_t kMost = (kLaunchThreads / (kRiskCandidates * kRiskWaves) - 1) * kRiskCandidates;
   auto launch = [&](auto kernel) {
-    kernel<<<static_cast<unsigned>(blocks), kRiskCandidates * kRiskWaves, 0, s>>>(
-        probabilities, output_projection, projected, margin, result, window, groups, length, first,
-        count, eps, accumulate);
+    for (int64_t done = 0; done < count; done += kMost) {
+      const int64_t here = std::min(kMost, count - done);
+      kernel<<<static_cast<unsigned>(ceil_div(here, kRiskCandidates)), kRiskCandidates * kRiskWaves,
+               0, s>>>(probabilities, output_projection, projected, margin, result + done, window,
+                       groups, length, first + done, here, eps, accumulate);
+    }
   };
   switch (groups) {
     case 1: launch(risk_kernel<1>); break;

@@ -93,6 +93,43 @@ def test_temporal_ops_across_row_and_window_sizes(device, window, groups, length
     assert torch.isnan(blind).all()  # exp(-inf - -inf), as the definition has it
 
 
+def test_temporal_risk_past_one_launch(device):
+    """2^28 candidates and some: more than one launch of 1,024-thread blocks of 64 candidates can
+    have (2^32 threads)."""
+    count, first = (1 << 28) + 77, 3
+    length = count + first
+    p = torch.full((1, 1, length), 0.25, device=device)
+    pv = torch.zeros((1, length), device=device)
+    marks = torch.tensor([0, 1, (1 << 28) - 65, (1 << 28) - 64, (1 << 28) - 63, (1 << 28) - 1,
+                          1 << 28, count - 1], device=device)
+    pv[0, first + marks] = torch.arange(1, 1 + marks.numel(), device=device).float()
+    margin = torch.tensor([2.0], device=device)
+    got = _C.temporal_risk(p, torch.zeros((1, 1), device=device), pv, margin, first, length, 1e-6)
+    few = _C.temporal_risk(p[..., :marks.numel()].contiguous(), torch.zeros((1, 1), device=device),
+                           pv[:, first + marks].contiguous(), margin, 0, marks.numel(), 1e-6)
+    assert torch.equal(got[marks], few) and (few > 0).all()
+    assert int(torch.count_nonzero(got)) == marks.numel()
+
+
+def test_temporal_probabilities_past_one_launch(device):
+    """2^22 rows and some of more than 4,096 keys: more than one launch of 1,024-thread rows can
+    have; equal, row by row, to a call of the last rows alone up to the order of the sums."""
+    rows, length, last = (1 << 22) + 5, 4097, 8
+    logits = torch.zeros((rows, 1, length), dtype=torch.float16, device=device)
+    logits[-last:] = rand((last, 1, length), torch.float16, device, 41)
+    pv = rand((1, length), torch.float32, device, 42)
+    qpos = torch.full((rows,), length, device=device)
+    kpos = torch.arange(length, device=device).float()
+    p, out = _C.temporal_probabilities(logits, pv, qpos, kpos, 1.0)
+    expect, out_expect = _C.temporal_probabilities(logits[-last:].contiguous(), pv, qpos[-last:],
+                                                   kpos, 1.0)
+    torch.testing.assert_close(p[-last:], expect, rtol=1e-5, atol=0)
+    torch.testing.assert_close(out[-last:], out_expect, rtol=1e-4, atol=1e-5)
+    torch.testing.assert_close(p[0], torch.full_like(p[0], 1 / length), rtol=1e-5, atol=0)
+    del logits, p  # 100 GB
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("chunk", [1, 7, 64, 1000])
 def test_temporal_head_scores_equals_the_operators(device, dtype, chunk):
