@@ -14,6 +14,7 @@ Two entry points:
 from __future__ import annotations
 
 import math
+import operator
 import time
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
@@ -76,10 +77,13 @@ def temporal_head_scores(queries, query_positions, keys, key_positions, values, 
     if query_chunk_size <= 0 or denominator_epsilon <= 0:
         raise ValueError("Chunk size and denominator epsilon must be positive")
     bytes_per_query = queries.shape[1] * keys.shape[0] * (keys.element_size() + 4)
-    chunk = min(query_chunk_size, max(1, (64 * 1024 ** 2) // bytes_per_query))
+    # operator.index: a chunk size that counts no queries (a float) is refused, as range() does
+    chunk = operator.index(min(query_chunk_size, max(1, (64 * 1024 ** 2) // bytes_per_query)))
+    if query_positions.ndim == 0 or (query_positions.shape[0] != queries.shape[0] > chunk):
+        raise RuntimeError("Invalid query positions")  # they are taken a chunk of rows at a time
     return (_temporal_module or _temporal()).temporal_head_scores(
         queries, query_positions, keys, key_positions, values, int(candidate_start),
-        int(candidate_end), margin_gradient, base_margin, float(denominator_epsilon), int(chunk))
+        int(candidate_end), margin_gradient, base_margin, float(denominator_epsilon), chunk)
 
 
 _temporal_module = None

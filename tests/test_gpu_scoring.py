@@ -168,6 +168,26 @@ def test_temporal_head_scores_equals_the_operators(device, dtype, chunk):
         torch.testing.assert_close(got, expect, rtol=0, atol=0, equal_nan=True)
 
 
+def test_temporal_head_scores_refuses_what_the_chunk_loop_refused(device):
+    """A chunk size that is no whole number, and positions that do not lie along the queries."""
+    window, length, dim = 20, 90, 64
+    arguments = lambda positions, chunk: (
+        rand((window, 2, dim), torch.bfloat16, device, 31), positions,
+        rand((length, dim), torch.bfloat16, device, 32), torch.arange(length, device=device),
+        rand((length, dim), torch.bfloat16, device, 33), 0, 60,
+        rand((2, dim), torch.float32, device, 34), torch.tensor(2.0), 1e-6, chunk)
+    positions = torch.arange(length - window, length, device=device)
+    with pytest.raises(TypeError):
+        scoring.temporal_head_scores(*arguments(positions, 8.0))
+    with pytest.raises(RuntimeError, match="Invalid query positions"):
+        scoring.temporal_head_scores(*arguments(positions[None], 8))
+    expect = scoring.temporal_head_scores(*arguments(positions, 8))
+    for accepted in (arguments(positions[:, None], np.int64(8)), arguments(positions, True + 7)):
+        assert torch.equal(scoring.temporal_head_scores(*accepted), expect)
+    whole = scoring.temporal_head_scores(*arguments(positions[None], 20))  # one chunk
+    torch.testing.assert_close(whole, expect, rtol=1e-5, atol=0)
+
+
 def test_temporal_risk_nonfinite(device):
     p = torch.full((3, 2, 10), 0.1, device=device)
     op = torch.zeros((3, 2), device=device)
