@@ -396,11 +396,11 @@ __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
 }
 
 // One coefficient row for each of several weights (pre-projection gradients of every layer).
-// grid: (column blocks, reduction groups, layers) of 256 threads, device [layers, 4] words (weight,
+// grid: (column blocks, groups, layers) of 256 threads, device [layers, 4] words (weight,
 // coefficients, gate or 0, out). A workgroup takes every row block b with b % groups = its group,
 // sums each as row_sum_kernel does and adds the sums in block order, as row_sum_reduce_kernel adds
-// its group: the same result bit for bit, with one partial row a group instead of one a block
-// (32 x 4096 x 4096 bf16: 8 MB of partials instead of 67 MB each way; 188 us instead of 223).
+// its group: with its groups (one partial row each) or a group a row block, the same result bit for
+// bit. layer_groups has the choice.
 template <typename T>
 __global__ __launch_bounds__(kRowSumThreads) void row_sum_layers_kernel(
     const int64_t* __restrict__ layer_table, int64_t vocab, int64_t dim, int64_t block_rows,
@@ -702,10 +702,34 @@ extern "C" int lr_pre_gradient(const float* post_gradient, const void* o_weight,
                        nullptr, gate, out, workspace, workspace_size, as_stream(stream));
 }
 
+namespace lr {
+namespace {
+
+// Groups of row_sum_layers_kernel: the reduction's where their workgroups fill the chip (from 192 on)
+// and take four row blocks each or more, else one a row block. us, one partial a group against one
+// a row block (bf16): 32 layers of 4096 x 4096 191 and 223 (8 MB of partials against 67), 6 layers
+// (192 workgroups) 31.8 and 34.7, 4 layers 27.8 and 24.4, one layer 25.3 and 9.4; 12 layers of
+// 2048 x 2048 19.2 and 19.6, 8 layers 16.4 and 14.3; 16 layers of 1024 x 1024 10.0 and 9.0.
+constexpr int64_t kFillingBlocks = 192;
+bool group_partials(int64_t layers, int64_t blocks, int64_t column_blocks) {
+  return layers * column_blocks * kReduceGroups >= kFillingBlocks && blocks >= 4 * kReduceGroups;
+}
+int64_t layer_groups(int64_t layers, int64_t blocks, int64_t width) {
+  return group_partials(layers, blocks, ceil_div(width, kRowSumColumns)) ? kReduceGroups : blocks;
+}
+
+}  // namespace
+}  // namespace lr
+
 extern "C" size_t lr_pre_gradient_layers_workspace_bytes(int64_t layers, int64_t hidden,
                                                          int64_t width) {
   if (layers <= 0 || hidden <= 0 || width <= 0) return 0;
-  return static_cast<size_t>(layers) * kReduceGroups * static_cast<size_t>(width) * sizeof(float);
+  const int64_t blocks = ceil_div(hidden, rows_per_block(hidden, width, 1));
+  int64_t rows = layers * layer_groups(layers, blocks, width);
+  // what fewer layers need fits too: the most of them that take a partial row a row block
+  const int64_t few = (kFillingBlocks - 1) / (ceil_div(width, kRowSumColumns) * kReduceGroups);
+  rows = std::max(rows, std::min(layers, few) * blocks);
+  return static_cast<size_t>(rows) * static_cast<size_t>(width) * sizeof(float);
 }
 
 extern "C" int lr_pre_gradient_layers(const int64_t* layer_table, int64_t layers, int64_t hidden,
@@ -724,7 +748,7 @@ extern "C" int lr_pre_gradient_layers(const int64_t* layer_table, int64_t layers
              "Row-sum workspace too small");
   const int64_t per_block = rows_per_block(hidden, width, 1);
   const int64_t blocks = ceil_div(hidden, per_block);
-  const int64_t groups = std::min<int64_t>(blocks, kReduceGroups);
+  const int64_t groups = layer_groups(layers, blocks, width);
   float* partial = static_cast<float*>(workspace);
   const hipStream_t s = as_stream(stream);
   int status = dispatch_weight(dtype, [&]<typename T>() {

@@ -122,6 +122,20 @@ def test_row_hidden_gradients_infinite_weights(device, rows, vocab, dim):
     assert torch.equal(torch.where(torch.isfinite(got), torch.zeros(()), got), expect)
 
 
+@pytest.mark.parametrize("layers,hidden,width", [(1, 2048, 2048), (11, 2048, 2048),
+                                                 (12, 2048, 2048), (6, 2100, 2056), (40, 300, 64)])
+def test_pre_gradients_layer_counts_match_per_layer(device, layers, hidden, width):
+    """Few layers (a partial row a row block), many (one a reduction group) and both sides of the
+    line between them: the per-layer call's sums in the same order, bit for bit."""
+    g = torch.Generator(device=device).manual_seed(layers)
+    weights = [torch.randn((hidden, width), generator=g, device=device).to(torch.bfloat16)
+               for _ in range(layers)]
+    posts = [torch.randn(hidden, generator=g, device=device) for _ in range(layers)]
+    batched = vjp.pre_gradients(posts, weights, width // 8, 8)
+    for post, weight, got in zip(posts, weights, batched):
+        assert torch.equal(got, vjp.pre_gradient(post, weight, width // 8, 8))
+
+
 def test_margins_given_and_argmax(device):
     rng = np.random.default_rng(3)
     logits = (rng.standard_normal((4, 128256)) * 3).astype(np.float32)

@@ -125,6 +125,17 @@ def test_pre_gradient_layers_width_bound_matches_per_layer_check():
     assert status == 1 and "at most 8192" in _lib.last_error()
 
 
+def test_pre_gradient_layers_workspace_holds_fewer_layers_too():
+    """A few layers get a partial row for each 32-row block (1,024 column and row blocks at most),
+    so that they fill the chip; a buffer sized for more layers holds what fewer need."""
+    size = _lib.load().lr_pre_gradient_layers_workspace_bytes
+    assert size(1, 4096, 4096) == 128 * 4096 * 4 and size(4, 4096, 4096) == 4 * 128 * 4096 * 4
+    assert size(32, 4096, 4096) == max(32 * 16, 5 * 128) * 4096 * 4
+    for hidden, width in [(4096, 4096), (2048, 2048), (1024, 1024), (100, 8192), (8192, 64)]:
+        sizes = [size(layers, hidden, width) for layers in range(1, 200)]
+        assert sizes == sorted(sizes)
+
+
 def test_batch_append_host_bounds_the_descriptor_table():
     """Descriptors in the launch's kernel arguments: at most 64 segments, rejected on the host
     before anything touches the device."""
