@@ -22,6 +22,7 @@
 //                        out = Z * gate (pre-projection gradient).
 
 #include <algorithm>
+#include <type_traits>
 
 #include "lr_common.hpp"
 #include "vjp_products.hpp"
@@ -71,8 +72,9 @@ __device__ __forceinline__ float load1(const T* p) {
   return static_cast<float>(*p);
 }
 
-// grid: ceil(V / 16) blocks of 256 threads. X rows [row0, row0 + RP) of [rows, D] in LDS.
-template <typename T, int RP>
+// grid: ceil(V / 16) blocks of 256 threads, or fewer that loop over W (LOOP). X rows [row0, row0 + RP)
+// of [rows, D] in LDS.
+template <typename T, int RP, bool LOOP>
 __global__ __launch_bounds__(kLogitThreads) void head_logits_kernel(
     const float* __restrict__ hidden, int64_t rows_here, int64_t dim, const T* __restrict__ weight,
     const T* __restrict__ bias, int64_t vocab, float* __restrict__ out, int64_t out_stride) {
@@ -84,9 +86,7 @@ __global__ __launch_bounds__(kLogitThreads) void head_logits_kernel(
       x[r * dim + i] = r < rows_here ? hidden[r * dim + i] : 0.f;
   __syncthreads();
   const int64_t chunks = dim / 8;
-  // Several rows: as many blocks as fit the chip, each staging X once for all its rows of W (a
-  // block per 16 rows of W stages half as many bytes of X again: eight f16 rows of 128,256 x 4096
-  // take 475 us against 967). One row: a block per 16 rows of W (188 against 217 us in a loop).
+  // Several rows: as many blocks as fit the chip, each staging X once for all its rows of W.
   for (int64_t block = blockIdx.x; block * kLogitRowsPerBlock < vocab; block += gridDim.x) {
   const int64_t v0 = block * kLogitRowsPerBlock + wave * kLogitRowsPerWave;
   const T* wrow[kLogitRowsPerWave];
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kLogitThreads) void head_logits_kernel(
         if (r < rows_here) out[r * out_stride + v] = bias ? acc[i][r] + b : acc[i][r];
     }
   }
-  if constexpr (RP == 1) return;
+  if constexpr (!LOOP) return;
   }
 }
 
@@ -367,6 +367,11 @@ __global__ __launch_bounds__(kRowSumThreads) void row_sum_kernel(RowSumArgs a) {
     float w[kRowUnroll][8];
 #pragma unroll
     for (int u = 0; u < kRowUnroll; ++u) load8<T>(weight + (v0 + k + u) * a.dim + col, w[u]);
+    // Left to itself the compiler takes the loads one by one into few registers where it has the
+    // sums of several rows to hold, each waited for (f32, four rows, 32,000 x 3072: 108 us, with all
+    // of them in flight 66; eight bf16 rows of 128,256 x 1000 143 and 78). f16 rows are faster so at
+    // the largest sizes (eight of 128,256 x 4096: 221 us, 244 with all in flight).
+    if constexpr (RP >= 4 && !std::is_same<T, _Float16>::value) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kRowUnroll; ++u)
 #pragma unroll
@@ -537,7 +542,7 @@ extern "C" int lr_head_logits(const float* hidden, int64_t rows, const void* wei
   if (int status = check_weight(dtype, vocab, dim, weight)) return status;
   LR_REQUIRE(rows > 0 && hidden && out, "Invalid hidden states");
   const hipStream_t s = as_stream(stream);
-  if (rows > 1 && takes_head_products(dtype, vocab, dim) && reinterpret_cast<uintptr_t>(hidden) % 16 == 0) {
+  if (rows > 1 && takes_head_products(dtype, rows, vocab, dim) && reinterpret_cast<uintptr_t>(hidden) % 16 == 0) {
     for (int64_t r0 = 0; r0 < rows; r0 += kProductRows) {
       const int64_t here = std::min<int64_t>(kProductRows, rows - r0);
       if (int status = launch_head_products(hidden + r0 * dim, here, weight, bias, vocab, dim,
@@ -551,23 +556,30 @@ extern "C" int lr_head_logits(const float* hidden, int64_t rows, const void* wei
     const int64_t here = std::min<int64_t>(per_pass, rows - r0);
     const int rp = row_pass(here);
     const int64_t lds = rp * dim * static_cast<int64_t>(sizeof(float));
-    const int64_t resident = 256 * std::min<int64_t>(8, (160 << 10) / lds);
-    int64_t blocks = ceil_div(vocab, kLogitRowsPerBlock);
-    if (rp > 1) blocks = std::min(blocks, resident);
+    // As many blocks as fit the chip, each staging X once and looping over W: a block per 16 rows of W
+    // stages half as many bytes of X again (eight f16 rows of 128,256 x 4096 475 us against 967, two of
+    // 32,000 x 8192 131 against 161). One row, and two short ones of 16 bits: a block per 16 rows (one
+    // row of 128,256 x 4096 188 us against 217; two f16 rows of 32,000 x 2048 30 against 35, the
+    // loop's registers costing occupancy).
+    constexpr int64_t kShortRows = 2048;
+    const int64_t blocks = ceil_div(vocab, kLogitRowsPerBlock);
+    const int64_t looping = std::min(blocks, 256 * std::min<int64_t>(8, (160 << 10) / lds));
     const int status = dispatch_weight(dtype, [&]<typename T>() {
       const T* w = static_cast<const T*>(weight);
       const T* b = static_cast<const T*>(bias);
-      auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kLogitThreads),
-                           static_cast<size_t>(rp) * dim * sizeof(float), s, hidden + r0 * dim,
-                           here, dim, w, b, vocab, out + r0 * vocab, vocab);
+      auto launch = [&](auto kernel, int64_t grid) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kLogitThreads),
+                           static_cast<size_t>(lds), s, hidden + r0 * dim, here, dim, w, b, vocab,
+                           out + r0 * vocab, vocab);
         return check_launch("head_logits");
       };
       switch (rp) {
-        case 1: return launch(head_logits_kernel<T, 1>);
-        case 2: return launch(head_logits_kernel<T, 2>);
-        case 4: return launch(head_logits_kernel<T, 4>);
-        default: return launch(head_logits_kernel<T, 8>);
+        case 1: return launch(head_logits_kernel<T, 1, false>, blocks);
+        case 2: return dim <= kShortRows && sizeof(T) == 2
+                           ? launch(head_logits_kernel<T, 2, false>, blocks)
+                           : launch(head_logits_kernel<T, 2, true>, looping);
+        case 4: return launch(head_logits_kernel<T, 4, true>, looping);
+        default: return launch(head_logits_kernel<T, 8, true>, looping);
       }
     });
     if (status) return status;
@@ -611,7 +623,7 @@ extern "C" size_t lr_row_sum_workspace_bytes(int64_t rows, int64_t vocab, int64_
   if (rows <= 0 || vocab <= 0 || dim <= 0) return 0;
   const int64_t pass = std::min<int64_t>(rows, 8);
   int64_t blocks = ceil_div(vocab, rows_per_block(vocab, dim, row_pass(pass)));
-  if (takes_column_products(LR_DTYPE_BF16, pass, dim))  // whichever kernel the weight's type takes
+  if (takes_column_products(LR_DTYPE_BF16, pass, vocab, dim))  // whichever kernel the weight's type takes
     blocks = std::max(blocks, ceil_div(vocab, column_product_block_rows(vocab, dim)));
   return static_cast<size_t>(blocks) * static_cast<size_t>(pass) * static_cast<size_t>(dim) *
          sizeof(float);
@@ -629,7 +641,7 @@ int weighted_rows(const void* weight, int dtype, int64_t vocab, int64_t dim, int
   LR_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "Workspace must be 16-byte aligned");
   for (int64_t r0 = 0; r0 < rows; r0 += 8) {
     const int64_t here = std::min<int64_t>(8, rows - r0);
-    const bool products = logits && takes_column_products(dtype, here, dim);
+    const bool products = logits && takes_column_products(dtype, here, vocab, dim);
     const int rp = row_pass(here);
     const int64_t per_block =
         products ? column_product_block_rows(vocab, dim) : rows_per_block(vocab, dim, rp);

@@ -295,11 +295,20 @@ void start_head(const float* hidden, int64_t rows, const void* weight, const voi
 }  // namespace
 
 // One row stays on the VALU, which already streams W at the card's rate (128,256 x 4096: 188 us
-// against 197 here; 8,001 x 2048: 12.5 against 15.4); two rows are faster here (206 against 276).
-// Hidden sizes: eight waves with whole 128-column stages, X's pieces in registers.
-bool takes_head_products(int dtype, int64_t vocab, int64_t dim) {
+// against 197 here; 8,001 x 2048: 12.5 against 15.4). Few rows need many weight rows to be worth
+// eight waves' start (us, VALU and here): two rows of 1,000 x 4096 11.4 and 22.3, of 8,001 x 3072
+// 18.2 and 22.0, of 32,000 x 1024 18.4 and 15.6, of 128,256 x 4096 261 and 205; three rows of 1,000 x
+// 5120 20.0 and 27.5, of 8,001 x 2048 18.0 and 13.6. Weight rows a multiple of 8 KB apart put the
+// 256 bytes a stage takes of each on the same memory channels, so two such rows change sides later
+// (32,000 x 4096 57 and 68). Hidden sizes: eight waves with whole 128-column stages, X's pieces in
+// registers.
+bool takes_head_products(int dtype, int64_t rows, int64_t vocab, int64_t dim) {
+  const int64_t least = rows <= 1   ? INT64_MAX
+                        : rows == 2 ? (dim % 4096 == 0 ? 65536 : 16384)
+                        : rows <= 4 ? 2048
+                                    : kHeadTile;
   return dtype == LR_DTYPE_BF16 && dim % 1024 == 0 && dim / 1024 <= kMaxHeadStages &&
-         vocab >= kHeadTile && vocab < (int64_t{1} << 30);
+         vocab >= least && vocab < (int64_t{1} << 30);
 }
 
 int launch_head_products(const float* hidden, int64_t rows, const void* weight, const void* bias,
@@ -315,9 +324,12 @@ int launch_head_products(const float* hidden, int64_t rows, const void* weight, 
 }
 
 // Up to two rows stay on the VALU (128,256 x 4096, two rows, with the statistics: 218 us against
-// 238); three rows of 8,001 x 2048 are 51 against 71, five of 50,001 x 3072 99 against 183.
-bool takes_column_products(int dtype, int64_t rows, int64_t dim) {
-  return dtype == LR_DTYPE_BF16 && rows > 2 && dim % kColumnTile == 0;
+// 238), and three or four against many weights (us, VALU and here: three rows of 32,000 x 2048 29.6 and
+// 37.2, of 128,256 x 4096 189 and 205, but of 8,001 x 2048 24.5 and 13.6; more rows of few weights
+// gain more than of many lose: five of 32,000 x 3072 60 and 42, of 128,256 x 4096 202 and 216).
+bool takes_column_products(int dtype, int64_t rows, int64_t vocab, int64_t dim) {
+  return dtype == LR_DTYPE_BF16 && dim % kColumnTile == 0 &&
+         (rows > 4 || (rows > 2 && vocab * dim < 60'000'000));
 }
 
 int64_t column_product_block_rows(int64_t vocab, int64_t dim) {

@@ -69,6 +69,14 @@ def test_head_logits_several_rows(device, rows, vocab, dim, bias):
         assert np.all(np.abs(got - expect) <= 1e-6 * scale)
 
 
+@pytest.mark.parametrize("rows,vocab,dim,bias", [
+    (8, 32, 1024, False), (5, 33, 2048, True), (3, 2047, 3072, False), (4, 2048, 3072, True),
+    (2, 16383, 1024, True), (2, 16384, 1024, False), (2, 16384, 4096, False)])
+def test_head_logits_both_sides_of_the_kernel_choice(device, rows, vocab, dim, bias):
+    """The vocabularies between which two, three and more rows change from one kernel to the other."""
+    test_head_logits_several_rows(device, rows, vocab, dim, bias)
+
+
 def test_head_logits_non_finite_rows_and_weights(device):
     """Infinities and NaN go where f32 arithmetic takes them, and nowhere else."""
     model, weight = model_with_head(device, 64, 1024, seed=40)
@@ -104,6 +112,14 @@ def test_row_hidden_gradients_several_rows(device, dtype, rows, vocab, dim):
     scale = np.abs(weight[t]) + (share / share.sum(axis=1, keepdims=True)) @ np.abs(weight)
     # the shares carry expf's and the division's f32 rounding, the sums chains of at most 32 + 251
     assert np.all(np.abs(got - expect) <= 2e-6 * scale)
+
+
+@pytest.mark.parametrize("rows,vocab,dim", [(3, 58593, 1024), (4, 58594, 1024), (3, 100, 1000)])
+def test_row_hidden_gradients_three_and_four_rows(device, rows, vocab, dim):
+    """Three and four rows on both sides of the weights at which they change kernels, bf16 and f32
+    (whose sums of four rows wait for a whole group of weight rows)."""
+    for dtype in (torch.bfloat16, torch.float32):
+        test_row_hidden_gradients_several_rows(device, dtype, rows, vocab, dim)
 
 
 @pytest.mark.parametrize("rows,vocab,dim", [(3, 17, 128), (8, 63, 256), (5, 513, 512)])
