@@ -98,14 +98,14 @@ def test_temporal_risk_past_one_launch(device):
     have (2^32 threads)."""
     count, first = (1 << 28) + 77, 3
     length = count + first
-    p = torch.full((1, 1, length), 0.25, device=device)
+    p = torch.full((9, 1, length), 0.25, device=device)
     pv = torch.zeros((1, length), device=device)
     marks = torch.tensor([0, 1, (1 << 28) - 65, (1 << 28) - 64, (1 << 28) - 63, (1 << 28) - 1,
                           1 << 28, count - 1], device=device)
     pv[0, first + marks] = torch.arange(1, 1 + marks.numel(), device=device).float()
     margin = torch.tensor([2.0], device=device)
-    got = _C.temporal_risk(p, torch.zeros((1, 1), device=device), pv, margin, first, length, 1e-6)
-    few = _C.temporal_risk(p[..., :marks.numel()].contiguous(), torch.zeros((1, 1), device=device),
+    got = _C.temporal_risk(p, torch.zeros((9, 1), device=device), pv, margin, first, length, 1e-6)
+    few = _C.temporal_risk(p[..., :marks.numel()].contiguous(), torch.zeros((9, 1), device=device),
                            pv[:, first + marks].contiguous(), margin, 0, marks.numel(), 1e-6)
     assert torch.equal(got[marks], few) and (few > 0).all()
     assert int(torch.count_nonzero(got)) == marks.numel()
