@@ -108,6 +108,59 @@ def test_long_prefill_many_chunks(device):
     check(run(device, q, k, v, meta, length, 1), q, k, v, cu, 1)
 
 
+def plan(segments, groups, length, keys, dim, dtype):
+    """[query rows of a tile, key splits] of a call (4 or 8 rows: the split-key kernel)."""
+    from code_for_iclr27_amd import _lib
+    out = np.zeros(2, np.int64)
+    _lib.call("lr_packed_attention_plan", segments, groups, length, keys, dim,
+              _lib.DTYPE_CODES[dtype], out.ctypes.data)
+    return out.tolist()
+
+
+# (segments, groups, queries, keys, dim): every form of the prefill kernel, as test_prefill_tile_forms
+# checks: 32- and 128-row tiles of each head dimension, keys in one part and split
+TILE_FORMS = {
+    (1, 4, 20, 20, 64): (32, False), (1, 4, 20, 1520, 64): (32, True),
+    (16, 8, 400, 400, 64): (128, False), (4, 8, 400, 500, 64): (128, True),
+    (1, 4, 20, 20, 128): (32, False), (1, 4, 200, 300, 128): (32, True),
+    (16, 8, 400, 400, 128): (128, False), (1, 8, 300, 1800, 128): (128, True),
+    (8, 6, 20, 20, 256): (32, False), (1, 8, 200, 200, 256): (32, True),
+    (16, 8, 131, 131, 256): (128, False), (8, 6, 64, 600, 256): (128, True),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", TILE_FORMS)
+def test_prefill_tile_forms(device, dtype, shape):
+    """Each form against the oracle (two further segments with fewer keys than queries and with
+    none, where the plan allows), its allocation-free call bit for bit the same, and a NaN and an
+    infinity in V at the last key: only the last query of its segment sees them."""
+    segments, groups, length, keys, dim = shape
+    rows, split = TILE_FORMS[shape]
+    chosen = plan(*shape, dtype)
+    assert chosen[0] == rows and (chosen[1] > 1) == split
+    lengths = [keys] * segments
+    if segments > 2:
+        lengths[1], lengths[2] = length - 7, 0
+    q, k, v, cu, meta = make(device, 1, segments, groups, length, dim, lengths, dtype, seed=27)
+    finite = run(device, q, k, v, meta, length, segments)
+    check(finite, q, k, v, cu, segments)
+    if rows == 32 or split:  # the unsplit 128-row calls are past that entry point's limit
+        fixed = through_the_abi(device, "lr_packed_attention_noalloc", q, k, v, meta, length,
+                                segments, dim ** -0.5)
+        assert torch.equal(fixed, finite)
+    bad = v.clone()
+    bad[keys - 1, 3], bad[keys - 1, dim - 1] = float("nan"), float("inf")
+    got = run(device, q, k, bad, meta, length, segments).view(length, segments, groups, dim)
+    finite = finite.view(length, segments, groups, dim)
+    columns = torch.tensor([3, dim - 1], device=device)
+    assert not torch.isfinite(got[-1, 0][..., columns]).any()
+    changed = torch.zeros_like(got, dtype=torch.bool)
+    changed[-1, 0] = torch.isin(torch.arange(dim, device=device), columns)
+    bound = ULP[got.dtype] * finite.float().abs() * 2 + 2e-4 * float(v.float().abs().max())
+    assert torch.all((got.float() - finite.float()).abs()[~changed] <= bound[~changed])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,kv_heads,groups,length,dim,lengths", [
     (1, 2, 3, 11, 128, [11, 43]),                    # 33 rows: a 32-row tile and one row more
@@ -116,27 +169,33 @@ def test_long_prefill_many_chunks(device):
     (1, 3, 4, 40, 64, [1040, 40, 7]),                # split keys; a segment shorter than the block
     (1, 2, 4, 40, 128, [2040, 0]),                   # split keys; an empty segment
     (1, 4, 6, 64, 256, [1064, 64, 300, 2064]),       # split keys, ragged
-    (2, 8, 8, 256, 128, [256] * 15 + [611]),         # tiles of 128 rows
+    (2, 8, 8, 256, 128, [256] * 15 + [611]),         # d128: tiles of 128 rows
     (2, 8, 8, 256, 64, [256] * 15 + [300]),
     (2, 6, 7, 131, 256, [131] * 11 + [700]),         # 917 rows: a ragged last tile
     (1, 1, 4, 300, 128, [4300]),                     # few units, long keys: many chunks
 ])
 def test_prefill_tiles(device, dtype, batch, kv_heads, groups, length, dim, lengths):
-    """The prefill kernel at the edges of its 32- and 128-row tiles, its 32-key stages and its key
-    chunks, and on segments with fewer keys than queries."""
+    """The prefill kernel at the edges of its tiles, its 32-key stages and its key chunks, and on
+    segments with fewer keys than queries (test_prefill_tile_forms runs each form by its plan)."""
     q, k, v, cu, meta = make(device, batch, kv_heads, groups, length, dim, lengths, dtype, seed=17)
     check(run(device, q, k, v, meta, length, kv_heads), q, k, v, cu, kv_heads)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("groups,length,dim,keys", [(4, 40, 64, 90), (4, 11, 128, 300),
-                                                    (6, 64, 256, 400), (1, 1, 64, 400)])
-def test_small_probabilities_keep_their_precision(device, dtype, groups, length, dim, keys):
+@pytest.mark.parametrize("segments,groups,length,dim,keys,rows", [
+    (2, 4, 40, 64, 90, 32), (16, 8, 400, 64, 400, 128), (2, 4, 40, 128, 2040, 32),
+    (16, 8, 400, 128, 400, 128), (8, 6, 20, 256, 20, 32), (16, 8, 131, 256, 131, 128),
+    (2, 4, 11, 128, 300, 8), (2, 1, 1, 64, 400, 4)])
+def test_small_probabilities_keep_their_precision(device, dtype, segments, groups, length, dim,
+                                                  keys, rows):
     """A dominant key with V = 0 and every other probability between 2^-27 and 2^-22 of it on
     large values: the outputs are sums of small P times V alone, as accurate as any other. In f32
     a small P carries its exponent's rounding (|exponent| < 32 here: 2^-20 ln 2, plus that of the
     scale and of the reference), under 2^-16 of the sum of P |V|."""
-    q, k, v, cu, meta = make(device, 1, 2, groups, length, dim, [keys, keys], dtype, seed=23)
+    if rows <= 8 or dim < 256:  # d256: f16 takes the other kernel on so few keys
+        assert plan(segments, groups, length, keys, dim, dtype)[0] == rows
+    q, k, v, cu, meta = make(device, 1, segments, groups, length, dim, [keys] * segments, dtype,
+                             seed=23)
     g = torch.Generator().manual_seed(24)
     q *= 2.0 ** -4  # the other dimensions' share of a score stays small
     q[..., 0] = 8.0
@@ -146,10 +205,10 @@ def test_small_probabilities_keep_their_precision(device, dtype, groups, length,
     v *= 2.0 ** 13
     k[cu[:-1]], v[cu[:-1]] = 0.0, 0.0
     arrays = [t.float().numpy() for t in (q, k, v)]
-    expect = oattention.packed_attention(*arrays, cu, 2)
-    total = oattention.packed_attention(*arrays[:2], np.abs(arrays[2]), cu, 2)
+    expect = oattention.packed_attention(*arrays, cu, segments)
+    total = oattention.packed_attention(*arrays[:2], np.abs(arrays[2]), cu, segments)
     assert 1e-4 < np.abs(expect).max() < 1
-    got = run(device, q, k, v, meta, length, 2).float().cpu().numpy()
+    got = run(device, q, k, v, meta, length, segments).float().cpu().numpy()
     # one rounding of the output (2^-25: half of f16's subnormal step)
     bound = ULP[dtype] * np.abs(expect) + 2.0 ** -16 * total + 2.0 ** -25
     assert np.all(np.abs(got - expect) <= bound), float((np.abs(got - expect) / bound).max())
@@ -235,7 +294,7 @@ def test_prefill_scales_through_the_abi(device, scale):
 
 @pytest.mark.parametrize("groups,length,dim,keys", [
     (4, 50, 64, [50, 120]),    # one-wave tiles
-    (8, 131, 128, [131] * 16), # tiles of four waves
+    (8, 131, 256, [131] * 16), # tiles of four waves
 ])
 def test_prefill_zero_scale_keeps_non_finite_scores(device, groups, length, dim, keys):
     """Scale 0 times an infinite or NaN score is NaN: the rows of such a query, and those that see

@@ -235,7 +235,7 @@ def test_pre_gradients_all_layers_match_per_layer(device, dtype, gated):
     for l in range(layers):
         single = vjp.pre_gradient(posts[l], weights[l], heads, dim, gates[l])
         assert batched[l].shape == (heads, dim)
-        torch.testing.assert_close(batched[l], single, rtol=0, atol=0)  # same kernels, same order
+        torch.testing.assert_close(batched[l], single, rtol=0, atol=0)  # same sums, same order
 
 
 def test_misaligned_weight_views_rejected(device):
