@@ -98,7 +98,9 @@ __device__ __forceinline__ SegmentKeys segment_keys(const AttnArgs& a, unsigned 
   return k;
 }
 
-template <typename T, int D, int R, int CH>
+// SEVERAL: several queries, of which a key may be hidden from some (a form of its own: the check
+// below, in every decode launch's instructions, cost 32 layers 2 us of 474).
+template <typename T, int D, int R, int CH, bool SEVERAL>
 __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attention_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128 || D == 256, "head dim");
   static_assert(R == 4 || R == 8, "rows per tile");
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(kAttnThreads, D == 256 ? 2 : 3) void packed_attenti
     }
     // A masked key's p is 0, and 0 * V is NaN for a non-finite V: a wave with a non-finite sum takes
     // its rows again, over the keys that each of them sees. (Every row of a decode call sees all.)
-    if (a.length > 1) {
+    if constexpr (SEVERAL) {
       float poison = 0.f;
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -494,8 +496,12 @@ bool takes_tiles(int64_t segments, int64_t groups, int64_t length, int64_t max_k
 
 template <typename T, int D, int R, int CH>
 int launch_attention(const AttnArgs& args, int64_t blocks, hipStream_t stream) {
-  hipLaunchKernelGGL((packed_attention_kernel<T, D, R, CH>), dim3(static_cast<unsigned>(blocks)),
-                     dim3(kAttnThreads), 0, stream, args);
+  auto attend = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, stream,
+                       args);
+  };
+  if (args.length > 1) attend(packed_attention_kernel<T, D, R, CH, true>);
+  else attend(packed_attention_kernel<T, D, R, CH, false>);
   if (int status = check_launch("packed_attention")) return status;
   if (args.splits == 1) return LR_OK;
   // Blocks each merging thread folds (PARTS = threads / (R * D / 8) threads share a row slice):
