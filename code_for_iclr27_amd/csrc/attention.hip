@@ -553,14 +553,15 @@ extern "C" size_t lr_packed_attention_workspace_bytes(int64_t segments, int64_t 
                                                       int64_t length, int64_t max_keys,
                                                       int64_t dim) {
   if (segments <= 0 || groups <= 0 || length <= 0 || max_keys < 0 || dim <= 0) return 0;
+  const size_t split_key = workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim);
+  if (length == 1) return split_key;
   // what either type needs: which kernel runs depends on it
-  size_t bytes = 0;
-  for (const int dtype : {LR_DTYPE_BF16, LR_DTYPE_F16})
-    bytes = std::max(bytes,
-                     takes_tiles(segments, groups, length, max_keys, dim, dtype)
-                         ? attention_tiles_bytes(plan_tiles(segments, groups, length, max_keys, dim), dim)
-                         : workspace_bytes(plan_attention(segments, groups, length, max_keys, dim), dim));
-  return bytes;
+  const bool bf16 = takes_tiles(segments, groups, length, max_keys, dim, LR_DTYPE_BF16);
+  const bool f16 = takes_tiles(segments, groups, length, max_keys, dim, LR_DTYPE_F16);
+  if (!bf16 && !f16) return split_key;
+  const size_t tiles =
+      attention_tiles_bytes(plan_tiles(segments, groups, length, max_keys, dim), dim);
+  return bf16 && f16 ? tiles : std::max(tiles, split_key);
 }
 
 extern "C" int lr_packed_attention_plan(int64_t segments, int64_t groups, int64_t length,
