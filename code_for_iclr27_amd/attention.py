@@ -4,10 +4,11 @@ src/lazy_recall/attention.py:15-35 (and its use by batch_attention.py:92-97).
 The reference hands the packed per-(request, KV head) segments to flash_attn's
 ``flash_attn_varlen_func`` (causal, softmax scale dim^-0.5, one KV head per segment, G query
 heads). Here the same call runs the HIP kernels of liblazyrecall_hip.so through
-``lr_packed_attention``: split-key flash decoding (QK^T on MFMA, P*V on the VALU) for decode, tiles
-of query rows with both products on MFMA for prefill (P in f32, as a sum of exact 16-bit pieces);
-f32 accumulation and the output rounded to the input dtype. There is no
-CPU path and no flash_attn dependency; CPU tensors are rejected.
+``lr_packed_attention``: split-key flash decoding (QK^T on MFMA, P*V on the VALU) for decode and a
+few queries, tiles of query rows with both products on MFMA for prefill (P in f32, as a sum of 16-bit
+pieces: exact in bf16, within 2^-60 of a row's largest in f16); f32 accumulation and the output
+rounded to the input dtype. There is no CPU path and no flash_attn dependency; CPU tensors are
+rejected.
 
 Forward only: the reference's audit step differentiates through this call with flash_attn's
 deterministic backward (attention.py:25-33); that backward is not part of this library, so a

@@ -591,7 +591,8 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
                      int64_t key_rows, const int32_t* cu_seqlens_k, int64_t batch,
                      int64_t kv_heads, int64_t groups, int64_t length, int64_t dim, int dtype,
                      int64_t max_keys, float scale, void* out, void* workspace,
-                     size_t workspace_size, void* stream, const void* pending_keys = nullptr, const void* pending_values = nullptr) {
+                     size_t workspace_size, void* stream, const void* pending_keys = nullptr,
+                     const void* pending_values = nullptr) {
   LR_REQUIRE(dtype == LR_DTYPE_BF16 || dtype == LR_DTYPE_F16,
              "FlashAttention only supports fp16 and bf16 data type");
   LR_REQUIRE((pending_keys == nullptr) == (pending_values == nullptr),
@@ -624,6 +625,8 @@ int packed_attention(const void* queries, int64_t q_batch_stride, int64_t q_head
              "Attention workspace too small");
   LR_REQUIRE(needed == 0 || reinterpret_cast<uintptr_t>(workspace) % 256 == 0,
              "Attention workspace must be 256-byte aligned");
+  // The split-key grid's limit, whichever kernel runs: a tile has at least as many rows, and a split
+  // tile plan has at most 32 MiB of states, so its grid is the smaller one.
   const int64_t blocks = plan.units * plan.splits;
   LR_REQUIRE(blocks < (int64_t{1} << 31), "Attention grid too large");
 
@@ -753,7 +756,7 @@ extern "C" int lr_packed_attention_noalloc(const void* queries, int64_t q_batch_
                                            void* stream) {
   clear_error();
   // The size check comes first and needs no HIP call; a call that needs no partial states
-  // (every segment within one key block) does not touch the scratch array at all.
+  // (every segment within one block of keys, whichever kernel runs) does not touch the scratch array.
   const int64_t segments =
       batch > 0 && kv_heads > 0 && batch <= (int64_t{1} << 31) / kv_heads ? batch * kv_heads : 0;
   // The limit is stated in the split-key plan's bytes whichever kernels run (plan_tiles keeps the

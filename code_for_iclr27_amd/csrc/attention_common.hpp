@@ -96,8 +96,9 @@ __device__ __forceinline__ T* output_row(const AttnArgs& a, unsigned seg, unsign
 }
 
 // A value and its copy in the lane 16 (32) away, in both lanes: the row swap of two registers that
-// hold it, no LDS round trip. (Inline assembly: this compiler's builtin returns its first result
-// twice. The wait states cover a vector instruction that has just written the operands.)
+// hold it, no LDS round trip. (Inline assembly: with the builtin, a bit cast of its second result as
+// a vector element takes the first one in this compiler. The wait states cover a vector instruction
+// that has just written the operands.)
 struct LanePair {
   float first, second;
 };

@@ -7,7 +7,8 @@
 // from HBM once, in its own dtype (bf16/f16/f32), and does the arithmetic in f32 as the
 // reference's `.float()` GEMMs do; the reference instead materialises f32 copies of 4096-row
 // weight chunks (written and re-read) and the [rows, V] probability matrix.
-// Several rows against a bf16 weight run on matrix cores instead (vjp_products.hip).
+// Several rows against a bf16 weight run on matrix cores instead where that is faster
+// (vjp_products.hip).
 //   head_logits_kernel   Y[r, v] = sum_d X[r, d] * W[v, d] (+ b[v]); a wave owns 4 rows of W,
 //                        lanes split D (16 B loads), X staged in LDS, one wave reduction per row.
 //   margin stats         per logits row: target (given, or the first argmax), competitor max M,
@@ -17,6 +18,8 @@
 //                        W, with c = softmax over the competitors (exp(l - M) / S, 0 at the
 //                        target) or a given coefficient vector; one thread per 8 columns of
 //                        a 2048-column block, 8 rows of W in flight per thread.
+//   row_sum_layers_kernel  the same with one given vector for each of several weights (every layer's
+//                        pre-projection gradient), coefficients by scalar loads.
 //   row_sum_reduce_kernel  the blocks' partials summed in a fixed order, then
 //                        out = (base - Z) * due (hidden gradient, base = W[target]) or
 //                        out = Z * gate (pre-projection gradient).

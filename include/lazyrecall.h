@@ -511,13 +511,14 @@ int lr_packed_attention_pending(const void* queries, int64_t q_batch_stride,
  * the workspace: the partial states live in one fixed array per device of
  * lr_packed_attention_scratch_bytes() bytes (16 MiB), held from the library's first use on that
  * device until the process ends. The call allocates and frees nothing. A call whose keys, split
- * as a decode call splits them (192 to 768 keys and up to 8 query rows a partial state), would
+ * as a decode call splits them (64 to 384 keys and up to 8 query rows a partial state), would
  * leave more than that size of partial states returns LR_ERR_INVALID with a message naming both
  * sizes, before anything is enqueued; prefill kernels keep theirs within it for every call
- * accepted. Every call on one device shares that
- * device's array and leaves its contents behind (none are needed at the next call): two calls
- * that can overlap in time on one device (different streams without an order between them)
- * race on it. The device is the one that owns `stream` (the current device for NULL). */
+ * accepted. Every call that needs a workspace shares its device's array and leaves its contents
+ * behind (none are needed at the next call): two such calls that can overlap in time on one
+ * device (different streams without an order between them) race on it; a call that needs none
+ * (every segment within one block of keys) does not touch it. The device is the one that owns
+ * `stream` (the current device for NULL). */
 size_t lr_packed_attention_scratch_bytes(void);
 int lr_packed_attention_noalloc(const void* queries, int64_t q_batch_stride,
                                 int64_t q_head_stride, int64_t q_query_stride, const void* keys,
