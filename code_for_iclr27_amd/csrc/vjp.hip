@@ -545,7 +545,8 @@ extern "C" int lr_head_logits(const float* hidden, int64_t rows, const void* wei
   if (int status = check_weight(dtype, vocab, dim, weight)) return status;
   LR_REQUIRE(rows > 0 && hidden && out, "Invalid hidden states");
   const hipStream_t s = as_stream(stream);
-  if (rows > 1 && takes_head_products(dtype, rows, vocab, dim) && reinterpret_cast<uintptr_t>(hidden) % 16 == 0) {
+  if (rows > 1 && takes_head_products(dtype, rows, vocab, dim) &&
+      reinterpret_cast<uintptr_t>(hidden) % 16 == 0) {
     for (int64_t r0 = 0; r0 < rows; r0 += kProductRows) {
       const int64_t here = std::min<int64_t>(kProductRows, rows - r0);
       if (int status = launch_head_products(hidden + r0 * dim, here, weight, bias, vocab, dim,

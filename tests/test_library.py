@@ -102,7 +102,8 @@ def test_attention_runs_the_faster_kernel_where_they_differ_much():
 
 def test_attention_workspace_covers_both_types():
     size = _lib.load().lr_packed_attention_workspace_bytes
-    for shape in [(8, 4, 2, 900, 64), (8, 4, 16, 4016, 128), (4, 6, 32, 532, 256), (4, 6, 32, 132, 256)]:
+    for shape in [(8, 4, 2, 900, 64), (8, 4, 16, 4016, 128), (4, 6, 32, 532, 256),
+                  (4, 6, 32, 132, 256)]:
         segments, groups, length, _, dim = shape
         for dtype in (_lib.LR_DTYPE_BF16, _lib.LR_DTYPE_F16):
             rows, splits = attention_plan(*shape, dtype)
