@@ -91,11 +91,13 @@ def attention_plan(segments, groups, length, keys, dim, dtype=_lib.LR_DTYPE_BF16
 def test_attention_runs_the_faster_kernel_where_they_differ_much():
     """Shapes at which one of the kernels measured at least a twentieth longer, most of them far."""
     f16 = _lib.LR_DTYPE_F16
-    split_key = [(4, 6, 8, 208, 256), (4, 6, 16, 516, 256), (4, 6, 8, 1008, 256), (8, 4, 2, 302, 64, f16),
-                 (8, 4, 32, 332, 64, f16), (4, 6, 8, 308, 256, f16), (8, 4, 1, 9000, 128)]
-    tiles = [(24, 4, 2, 4002, 128), (24, 4, 4, 4004, 128), (8, 4, 8192, 8192, 128), (8, 4, 333, 333, 64), (8, 4, 333, 333, 64, f16),
-             (4, 6, 1000, 5000, 256), (4, 6, 1000, 5000, 256, f16), (8, 4, 8, 4008, 64),
-             (24, 4, 8, 2861, 128), (8, 4, 32, 100, 64), (8, 4, 128, 1128, 128)]
+    split_key = [(4, 6, 8, 208, 256), (4, 6, 16, 516, 256), (4, 6, 8, 1008, 256),
+                 (8, 4, 2, 302, 64, f16), (8, 4, 32, 332, 64, f16), (4, 6, 8, 308, 256, f16),
+                 (8, 4, 1, 9000, 128)]
+    tiles = [(24, 4, 2, 4002, 128), (24, 4, 4, 4004, 128), (8, 4, 8192, 8192, 128),
+             (8, 4, 333, 333, 64), (8, 4, 333, 333, 64, f16), (4, 6, 1000, 5000, 256),
+             (4, 6, 1000, 5000, 256, f16), (8, 4, 8, 4008, 64), (24, 4, 8, 2861, 128),
+             (8, 4, 32, 100, 64), (8, 4, 128, 1128, 128)]
     assert all(attention_plan(*shape)[0] <= 8 for shape in split_key)
     assert all(attention_plan(*shape)[0] >= 32 for shape in tiles)
 
